@@ -617,10 +617,17 @@ __device__ __forceinline__ void stage_item(const StageArgs& a, int tile_x, int t
     if (DEFER && zp >= 0) update(zp, fpend, zpend);
 }
 
+// First plane of z chunk k of nch over the planes 2 .. nPz-1: the chunks hold
+// q = (nPz-2)/nch planes, the first (nPz-2) mod nch of them one more.
+__host__ __device__ __forceinline__ int chunk_begin(int nPz, int nch, int q, int k)
+{
+    const int r = nPz - 2 - q * nch;
+    return 2 + k * q + (k < r ? k : r);
+}
+
 // One stage of one domain: block -> (tile, z chunk) work item.  With
 // xcd_remap, consecutive tiles go to the same XCD (blocks are dealt to the 8
-// XCDs round-robin) so halo re-reads hit its L2.  Chunk k covers the planes
-// 2 + k*zchunk .. (the last chunk runs to nPz-1).
+// XCDs round-robin) so halo re-reads hit its L2.
 template <typename T, bool MAG, bool ROT, int STAGE, int WAVES, bool ONE_BARRIER, bool DEFER,
           bool EXT = false, int EXTM = EXT_INTERIOR, bool S32 = false>
 __global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, int zchunk, int nch,
@@ -636,8 +643,8 @@ __global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, i
     const int rest = logical / ntx;
     const int tile_y = rest % nty;
     const int chunk = rest / nty;
-    const int zb = 2 + chunk * zchunk;
-    const int ze = chunk == nch - 1 ? a.g.nPz : zb + zchunk;
+    const int zb = chunk_begin(a.g.nPz, nch, zchunk, chunk);
+    const int ze = chunk_begin(a.g.nPz, nch, zchunk, chunk + 1);
     CflAcc cfl;   // stage 3: TSTEP of the next step on the new state
     stage_item<T, MAG, ROT, STAGE, ONE_BARRIER, DEFER, EXT, EXTM, S32>(a, tile_x, tile_y, zb, ze, lds, cfl);
     if (STAGE == 3 && a.cfl_parts) {
@@ -652,12 +659,10 @@ struct StreamPlan {
     int zchunk, nchunks, ntx, nty, nblocks, xcd_remap;
 };
 
-// Work decomposition of one domain: 32 x 8 tiles times z chunks of at least
-// 8 planes (the last chunk takes the remainder), about target_blocks items.
-// The launch is fastest when its blocks fill the device's resident slots
-// once (no second round, no chunk-overlap planes beyond what that needs), so
-// the caller passes the resident block count of the kernel variant.
-inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024)
+// Work decomposition of one domain: 32 x 8 tiles times the z chunks that make
+// about target_blocks items (at least min_planes planes each), the planes
+// dealt evenly to the chunks.
+inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024, int min_planes = 1)
 {
     StreamPlan p;
     p.ntx = (g.nPx + STX - 1) / STX;
@@ -665,7 +670,7 @@ inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024)
     const int nint = g.nPz - 2;
     const int tiles = p.ntx * p.nty;
     int nch = (target_blocks + tiles - 1) / tiles;
-    const int maxch = nint / 8 > 0 ? nint / 8 : 1;
+    const int maxch = nint / min_planes > 0 ? nint / min_planes : 1;
     if (nch > maxch) nch = maxch;
     if (nch < 1) nch = 1;
     p.zchunk = nint / nch;
@@ -673,6 +678,41 @@ inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024)
     p.nblocks = tiles * p.nchunks;
     p.xcd_remap = (p.nblocks % 8 == 0) ? 1 : 0;
     return p;
+}
+
+// Blocks of one launch on a device that holds `resident` of them at once: the
+// z split whose blocks fill whole rounds of the resident slots.  A chunk of p
+// planes costs about p + 2 plane times (its two overlap planes), so R rounds
+// cost R * (p + 2), p the planes of the longest chunk that R rounds allow;
+// the fewest plane times win, over at most 8 rounds (which bounds the TSTEP
+// partial records) and chunks of at most max_planes planes (0: no limit)
+// where a split has them.  Measured on MI355X, FP64 MHD, us a step (chunks:
+// time): 64^3 4: 209, 16: 108, 31: 101, 62: 111; 96x96x64 12: 172, 14 (one
+// full round): 159, 15: 197, 28: 187; 192x192x96 3: 655, 4 (a second round
+// of 64 blocks): 752, 7 (two full rounds): 614, 10: 646; 256x256x128 1: 1556,
+// 2: 1265, 4: 1293.  Before, chunks held at least 8 planes, the last one the
+// remainder as well.
+inline int round_blocks(const Geom& g, int resident, int max_planes)
+{
+    const int tiles = ((g.nPx + STX - 1) / STX) * ((g.nPy + STY - 1) / STY);
+    const int nint = g.nPz - 2;
+    const int64_t r0 = ((int64_t)tiles + resident - 1) / resident;
+    const int64_t r1 = r0 > 8 ? r0 : 8;
+    int best_n = 1;
+    int64_t best = -1;
+    for (int pass = max_planes > 0 ? 0 : 1; pass < 2 && best < 0; ++pass)
+        for (int64_t r = r0; r <= r1; ++r) {
+            int64_t n = r * resident / tiles;
+            if (n > nint) n = nint;
+            const int64_t planes = (nint + n - 1) / n;
+            if (pass == 0 && planes > max_planes) continue;
+            const int64_t cost = ((tiles * n + resident - 1) / resident) * (planes + 2);
+            if (best < 0 || cost < best) {
+                best = cost;
+                best_n = (int)n;
+            }
+        }
+    return tiles * best_n;
 }
 
 // Launch of one interior stage.  sched bit 0: one barrier per plane

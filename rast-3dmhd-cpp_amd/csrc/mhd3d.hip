@@ -350,17 +350,6 @@ static int variant_resident(const mhd3d_ctx* ctx, int w, int sc)
     return resident_blocks(fn, STX * STY);
 }
 
-// Blocks of one streaming launch: the resident blocks, or (planes > 0) z
-// chunks of at most `planes` planes in rounds of them -- at most 8 rounds,
-// which bounds the TSTEP partial records.
-static int launch_blocks(const mhd3d_ctx* ctx, int resident, int planes)
-{
-    if (planes <= 0) return resident;
-    const StreamPlan one = stream_plan(ctx->g, 1);
-    const int want = one.ntx * one.nty * ((ctx->g.nPz - 2 + planes - 1) / planes);
-    return std::max(resident, std::min(want, 8 * resident));
-}
-
 extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
 {
     if (!out) return MHD3D_EINVAL;
@@ -472,18 +461,18 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
             }
         }
     const char* tb = std::getenv("MHD3D_TARGET_BLOCKS");
-    if (tb && std::atoi(tb) >= 1) ctx->target_blocks = std::atoi(tb);
+    if (tb && std::atoi(tb) >= 1)   // an override in z chunks of at least 8 planes
+        ctx->target_blocks = stream_plan(g, std::atoi(tb), 8).nblocks;
     const char* fc = std::getenv("MHD3D_FUSE_CFL");
     if (fc && std::atoi(fc) == 0) ctx->fuse_cfl = false;
     if (ctx->mixed) ctx->kernel_mode = 0;   // the mixed form has only the streaming kernel
     if (ctx->target_blocks == 0) {
         const int fm = ctx->mixed ? 1 : 0, ph = desc->flag_lMag ? 1 : 0;
         // FP64: z chunks of at most 64 planes (MI355X, FP64 MHD 512x512x256
-        // stage kernel: one chunk 3.47 ms, two 3.40, four 3.35, eight 3.74;
-        // 256x256x128 is best at its resident count, two chunks of 63); the
-        // mixed form: one round of its resident blocks (its best)
-        ctx->target_blocks = launch_blocks(ctx, variant_resident(ctx, ctx->tune_waves[fm][ph], ctx->tune_sched[fm][ph]),
-                                           ctx->mixed ? 0 : 64);
+        // stage kernel: one chunk 3.47 ms, two 3.40, four 3.35, eight 3.74);
+        // the mixed form is best with the longest chunks its rounds allow
+        ctx->target_blocks = round_blocks(g, variant_resident(ctx, ctx->tune_waves[fm][ph], ctx->tune_sched[fm][ph]),
+                                          ctx->mixed ? 0 : 64);
     }
     *out = ctx;
     return MHD3D_OK;
@@ -1474,7 +1463,7 @@ extern "C" int mhd3d_autotune(mhd3d_ctx* ctx, int steps, double* report, int* nc
             for (int ip = 0; ip < 3 && !rc; ++ip) {
                 ctx->tune_waves[fm][ph] = wv[iw];
                 ctx->tune_sched[fm][ph] = is;
-                ctx->target_blocks = launch_blocks(ctx, variant_resident(ctx, wv[iw], is), planes[ip]);
+                ctx->target_blocks = round_blocks(ctx->g, variant_resident(ctx, wv[iw], is), planes[ip]);
                 ctx->dt_ready = false;   // the partial records follow the launch size
                 double dt = 0.0;
                 int r = step_core(ctx, 1, 0, &dt);   // warm-up
@@ -1816,7 +1805,7 @@ static int ens_build(mhd3d_ensemble* e)
         // as alone)
         const bool ext_interior = e->mixed ? c->ext : ext_variant(c->xa.flags) != EXTV_NONE;
         if (needs_prepass(c)) e->prepass = true;
-        StreamPlan p = stream_plan(g, 256);
+        StreamPlan p = stream_plan(g, 256, 8);
         if (e->chunk > 0) {
             const int nint = g.nPz - 2;
             p.nchunks = nint / e->chunk > 0 ? nint / e->chunk : 1;
@@ -1828,8 +1817,8 @@ static int ens_build(mhd3d_ensemble* e)
                 for (int tx = 0; tx < p.ntx; ++tx) {
                     WorkItem w{};
                     w.member = m; w.flags = flags; w.tile_x = tx; w.tile_y = ty;
-                    w.zb = 2 + ch * p.zchunk;
-                    w.ze = ch == p.nchunks - 1 ? g.nPz : w.zb + p.zchunk;
+                    w.zb = chunk_begin(g.nPz, p.nchunks, p.zchunk, ch);
+                    w.ze = chunk_begin(g.nPz, p.nchunks, p.zchunk, ch + 1);
                     w.part = part++;
                     (ext_interior ? items_x : items).push_back(w);
                 }
