@@ -63,6 +63,6 @@ struct WallItem;
 // kernel is for occupancy queries.
 const void* ext_ens_fn_s32();
 void ext_ens_stage_s32(int stage, const StageArgs* args, const WorkItem* items, int nitems, int grid_int,
-                       const WallItem* walls, int nwalls, int grid_wall, hipStream_t s);
+                       const WallItem* walls, int nwalls, int grid_wall, bool full_walls, hipStream_t s);
 
 }  // namespace mhd

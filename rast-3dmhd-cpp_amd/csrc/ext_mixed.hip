@@ -109,7 +109,7 @@ const void* ext_ens_fn_s32()
 }
 
 void ext_ens_stage_s32(int stage, const StageArgs* args, const WorkItem* items, int nitems, int grid_int,
-                       const WallItem* walls, int nwalls, int grid_wall, hipStream_t s)
+                       const WallItem* walls, int nwalls, int grid_wall, bool full_walls, hipStream_t s)
 {
     if (nitems > 0) {
         const dim3 blk(STX, STY, 1);
@@ -117,12 +117,7 @@ void ext_ens_stage_s32(int stage, const StageArgs* args, const WorkItem* items, 
         else if (stage == 2) ensemble_stage_ext_kernel<2, true><<<grid_int, blk, 0, s>>>(args, items, nitems);
         else ensemble_stage_ext_kernel<3, true><<<grid_int, blk, 0, s>>>(args, items, nitems);
     }
-    if (nwalls > 0) {
-        const dim3 wblk(64, 4, 1);
-        if (stage == 1) ensemble_wall_kernel<double, 1, true, true><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
-        else if (stage == 2) ensemble_wall_kernel<double, 2, true, true><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
-        else ensemble_wall_kernel<double, 3, true, true><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
-    }
+    if (nwalls > 0) launch_ens_walls<double, true, true>(stage, full_walls, grid_wall, args, walls, nwalls, s);
 }
 
 }  // namespace mhd

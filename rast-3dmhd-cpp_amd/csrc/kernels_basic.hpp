@@ -528,13 +528,23 @@ __device__ __forceinline__ void bcon_point(const Phys& c, const Metric& m, const
 // at stages 2-3; the update, BCON and the Z register in FP64; BCON reads the
 // new inward planes from the FP32 copy at stages 1-2 and from the FP64 state
 // at stage 3).
-template <typename T, bool MAG, bool ROT, int STAGE, bool EXT = false, bool S32 = false>
+// FULL = false: only RO (and BX, BY) of the wall are advanced by their
+// fluxes.  BCON replaces RU, RV, RW, TT and BZ there from planes inward and
+// constants, and their Z register is read by nothing but the update BCON
+// replaces, so their fluxes -- the viscous, conduction, heating and Lorentz
+// terms of the wall -- have no reader.  FULL = true where one has: iTCon 3,
+// whose top wall keeps the TT its flux gives, and lShr, whose FT register
+// carries over (walls_full).  us a wall launch, every flux -> these,
+// FP64 MHD (MI355X, rocprofv3, stages 1 / 2): 32^3 12.1 / 12.4 -> 5.2 / 6.3,
+// 64^3 13.9 / 14.4 -> 5.8 / 7.3, 256x256x128 28.5 / 29.7 -> 14.2 / 15.0.
+template <typename T, bool MAG, bool ROT, int STAGE, bool EXT = false, bool S32 = false, bool FULL = true>
 __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, bool top, CflAcc& cfl)
 {
     constexpr bool F64 = std::is_same<T, double>::value;
     static_assert(F64 || !EXT, "the off-default branches are evaluated in FP64");
     static_assert(F64 || !S32, "S32: FP64 fluxes from the mixed form's FP32 copies");
     constexpr int NF = MAG ? NF_MAG : NF_HYDRO;
+    auto kept = [](int f) { return FULL || f == 3 || f == 5 || f == 6; };
     const int z = top ? 1 : a.g.nPz;
     const int zi1 = top ? z + 1 : z - 1;   // first plane inward
     const int zi2 = top ? z + 2 : z - 2;   // second plane inward
@@ -555,7 +565,7 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
                 flux_point<MAG, ROT, 1, double, false, EXT>(acc, a.c, pm, o, &e);
             else
                 flux_point<MAG, ROT, 2, double, false, EXT>(acc, a.c, pm, o, &e);
-            if constexpr (EXT) {
+            if constexpr (EXT && FULL) {
                 if (a.x.flags & EXT_SHR) a.x.ft[(int64_t)z * a.g.plane + (int64_t)y * a.g.pitch + x] = o.FT;
             }
         };
@@ -585,9 +595,10 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
     const int64_t i1 = (int64_t)zi1 * a.g.plane + row;
     const int64_t i2 = (int64_t)zi2 * a.g.plane + row;
     const int64_t fs = a.g.fs;
-    double un[NF];
+    double un[NF] = {};
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
+        if (!kept(f)) continue;
         const double zin = STAGE == 1 ? a.Uin[f * fs + i] : a.Z[f * fs + i];
         un[f] = zin + cg * fsel(o, f);
     }
@@ -607,7 +618,7 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
             a.Uout[f * fs + i] = un[f];
         else
             a.Uout32[f * fs + i] = float(un[f] - bg_sub(a, f, z));
-        if (STAGE < 3) a.Z[f * fs + i] = un[f] + cz * fsel(o, f);
+        if (STAGE < 3 && kept(f)) a.Z[f * fs + i] = un[f] + cz * fsel(o, f);
     }
     if (STAGE == 3 && a.cfl_parts) {
         double wp[5], up;
@@ -623,7 +634,7 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
 // for three waves per SIMD (FP64) or two (the mixed form's deviation
 // stencils), so the register allocator keeps the occupancy; the off-default
 // variant needs the registers of one wave.
-template <typename T, bool MAG, bool ROT, int STAGE, bool EXT = false, bool S32 = false>
+template <typename T, bool MAG, bool ROT, int STAGE, bool EXT = false, bool S32 = false, bool FULL = true>
 __global__ void __launch_bounds__(256, EXT ? 1 : (sizeof(T) == 4 ? 2 : 3)) stage_wall_kernel(StageArgs a)
 {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -633,7 +644,7 @@ __global__ void __launch_bounds__(256, EXT ? 1 : (sizeof(T) == 4 ? 2 : 3)) stage
     // every thread reaches the block reduction below; threads outside the
     // domain only contribute the identity
     CflAcc cfl;
-    if (x < a.g.nPx && y < a.g.nPy) wall_point<T, MAG, ROT, STAGE, EXT, S32>(a, x, y, top, cfl);
+    if (x < a.g.nPx && y < a.g.nPy) wall_point<T, MAG, ROT, STAGE, EXT, S32, FULL>(a, x, y, top, cfl);
     if (STAGE == 3 && a.cfl_parts) {
         const int b = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
         cfl_block_reduce(cfl, a.cfl_parts, a.cfl_base + b);

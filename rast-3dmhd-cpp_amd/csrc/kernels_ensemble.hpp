@@ -132,7 +132,9 @@ __global__ void __launch_bounds__(256, 1)
 // the members with off-default branches (FP64 fluxes; S32: of the mixed
 // form), in a list and a launch of their own so the others keep the smaller
 // register budget.
-template <typename T, int STAGE, bool EXT = false, bool S32 = false>
+// FULL = false: every member's walls advance only the fields BCON leaves
+// (wall_point), which no rotation term touches.
+template <typename T, int STAGE, bool EXT, bool S32, bool FULL>
 __global__ void __launch_bounds__(256)
     ensemble_wall_kernel(const StageArgs* __restrict__ args, const WallItem* __restrict__ items,
                          int nitems)
@@ -145,14 +147,35 @@ __global__ void __launch_bounds__(256)
         CflAcc cfl;
         if (x < a.g.nPx && y < a.g.nPy) {
             const bool top = w.top != 0;
-            switch (w.flags & 3) {
-            case 0: wall_point<T, false, false, STAGE, EXT, S32>(a, x, y, top, cfl); break;
-            case 1: wall_point<T, true, false, STAGE, EXT, S32>(a, x, y, top, cfl); break;
-            case 2: wall_point<T, false, true, STAGE, EXT, S32>(a, x, y, top, cfl); break;
-            default: wall_point<T, true, true, STAGE, EXT, S32>(a, x, y, top, cfl); break;
+            switch (w.flags & (FULL ? 3 : 1)) {
+            case 0: wall_point<T, false, false, STAGE, EXT, S32, FULL>(a, x, y, top, cfl); break;
+            case 1: wall_point<T, true, false, STAGE, EXT, S32, FULL>(a, x, y, top, cfl); break;
+            case 2:
+                if constexpr (FULL) wall_point<T, false, true, STAGE, EXT, S32, FULL>(a, x, y, top, cfl);
+                break;
+            default:
+                if constexpr (FULL) wall_point<T, true, true, STAGE, EXT, S32, FULL>(a, x, y, top, cfl);
+                break;
             }
         }
         if (STAGE == 3 && a.cfl_parts) cfl_block_reduce(cfl, a.cfl_parts, w.part);
+    }
+}
+
+// The wall launch of one stage over the members of a list.
+template <typename T, bool EXT, bool S32>
+static void launch_ens_walls(int stage, bool full, int grid, const StageArgs* args, const WallItem* walls, int n,
+                             hipStream_t s)
+{
+    const dim3 blk(64, 4, 1);
+    if (full) {
+        if (stage == 1) ensemble_wall_kernel<T, 1, EXT, S32, true><<<grid, blk, 0, s>>>(args, walls, n);
+        else if (stage == 2) ensemble_wall_kernel<T, 2, EXT, S32, true><<<grid, blk, 0, s>>>(args, walls, n);
+        else ensemble_wall_kernel<T, 3, EXT, S32, true><<<grid, blk, 0, s>>>(args, walls, n);
+    } else {
+        if (stage == 1) ensemble_wall_kernel<T, 1, EXT, S32, false><<<grid, blk, 0, s>>>(args, walls, n);
+        else if (stage == 2) ensemble_wall_kernel<T, 2, EXT, S32, false><<<grid, blk, 0, s>>>(args, walls, n);
+        else ensemble_wall_kernel<T, 3, EXT, S32, false><<<grid, blk, 0, s>>>(args, walls, n);
     }
 }
 

@@ -921,20 +921,23 @@ static void launch_stage_t(mhd3d_ctx* ctx, const StageArgs& a)
     }
 }
 
-template <bool MAG, bool ROT, int STAGE>
+// Whether a wall flux other than those of RO, BX, BY has a reader (wall_point).
+static bool walls_full(const mhd3d_desc& d) { return d.flag_iTCon == 3 || d.flag_lShr; }
+
+template <bool MAG, bool ROT, int STAGE, bool FULL>
 static void launch_wall_t(mhd3d_ctx* ctx, const StageArgs& a)
 {
     const Geom& g = ctx->g;
     dim3 blk(64, 4, 1);
     dim3 grd((g.nPx + 63) / 64, (g.nPy + 3) / 4, 2);
     if (ctx->mixed && ctx->ext)
-        stage_wall_kernel<double, MAG, ROT, STAGE, true, true><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, true, true, FULL><<<grd, blk, 0, ctx->stream>>>(a);
     else if (ctx->mixed)
-        mixed_wall(MAG, ROT, STAGE, a, grd, blk, ctx->stream);
+        mixed_wall(MAG, ROT, STAGE, FULL, a, grd, blk, ctx->stream);
     else if (ctx->ext)
-        stage_wall_kernel<double, MAG, ROT, STAGE, true><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, true, false, FULL><<<grd, blk, 0, ctx->stream>>>(a);
     else
-        stage_wall_kernel<double, MAG, ROT, STAGE><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, false, false, FULL><<<grd, blk, 0, ctx->stream>>>(a);
 }
 
 template <int STAGE>
@@ -947,10 +950,13 @@ static void launch_stage_k(mhd3d_ctx* ctx, const StageArgs& a, bool wall)
         else if (rot) launch_stage_t<false, true, STAGE>(ctx, a);
         else launch_stage_t<false, false, STAGE>(ctx, a);
     } else {
-        if (mag && rot) launch_wall_t<true, true, STAGE>(ctx, a);
-        else if (mag) launch_wall_t<true, false, STAGE>(ctx, a);
-        else if (rot) launch_wall_t<false, true, STAGE>(ctx, a);
-        else launch_wall_t<false, false, STAGE>(ctx, a);
+        if (!walls_full(ctx->d)) {   // no rotation term in the fluxes kept
+            if (mag) launch_wall_t<true, false, STAGE, false>(ctx, a);
+            else launch_wall_t<false, false, STAGE, false>(ctx, a);
+        } else if (mag && rot) launch_wall_t<true, true, STAGE, true>(ctx, a);
+        else if (mag) launch_wall_t<true, false, STAGE, true>(ctx, a);
+        else if (rot) launch_wall_t<false, true, STAGE, true>(ctx, a);
+        else launch_wall_t<false, false, STAGE, true>(ctx, a);
     }
 }
 
@@ -1632,6 +1638,7 @@ struct mhd3d_ensemble {
     FinishArgs* d_fin = nullptr;
     int nitems = 0, nwalls = 0, nitems_x = 0, nwalls_x = 0;
     int grid_int = 0, grid_wall = 0, grid_x = 0, grid_wall_x = 0;
+    bool full_walls = false, full_walls_x = false;   // some member's walls need every flux (walls_full)
     bool prepass = false;              // some member needs plane means / the relaxation pass
     int waves = 1, sched = 0, chunk = 0;   // kernel variant; chunk: planes per item (0 = auto)
     int parity = 0;                    // FP64: register parity of the step tables
@@ -1703,17 +1710,12 @@ static void ens_stage(const mhd3d_ensemble* e, int k, const StageArgs* args)
         else if (k == 2) ensemble_stage_ext_kernel<2><<<e->grid_x, blk, 0, e->stream>>>(args, e->d_items_x, e->nitems_x);
         else ensemble_stage_ext_kernel<3><<<e->grid_x, blk, 0, e->stream>>>(args, e->d_items_x, e->nitems_x);
     }
-    dim3 wblk(64, 4, 1);
     if (e->nwalls > 0) {
-        if (k == 1) ensemble_wall_kernel<T, 1><<<e->grid_wall, wblk, 0, e->stream>>>(args, e->d_walls, e->nwalls);
-        else if (k == 2) ensemble_wall_kernel<T, 2><<<e->grid_wall, wblk, 0, e->stream>>>(args, e->d_walls, e->nwalls);
-        else ensemble_wall_kernel<T, 3><<<e->grid_wall, wblk, 0, e->stream>>>(args, e->d_walls, e->nwalls);
+        launch_ens_walls<T, false, false>(k, e->full_walls, e->grid_wall, args, e->d_walls, e->nwalls, e->stream);
     }
     if (e->nwalls_x > 0) {
-        const WallItem* wx = e->d_walls_x;
-        if (k == 1) ensemble_wall_kernel<double, 1, true><<<e->grid_wall_x, wblk, 0, e->stream>>>(args, wx, e->nwalls_x);
-        else if (k == 2) ensemble_wall_kernel<double, 2, true><<<e->grid_wall_x, wblk, 0, e->stream>>>(args, wx, e->nwalls_x);
-        else ensemble_wall_kernel<double, 3, true><<<e->grid_wall_x, wblk, 0, e->stream>>>(args, wx, e->nwalls_x);
+        launch_ens_walls<double, true, false>(k, e->full_walls_x, e->grid_wall_x, args, e->d_walls_x, e->nwalls_x,
+                                              e->stream);
     }
 }
 
@@ -1797,9 +1799,11 @@ static int ens_build(mhd3d_ensemble* e)
     std::vector<WallItem> walls, walls_x;
     std::vector<FinishArgs> fin(e->n);
     e->prepass = false;
+    e->full_walls = e->full_walls_x = false;
     for (int m = 0; m < e->n; ++m) {
         mhd3d_ctx* c = e->mem[m];
         const Geom& g = c->g;
+        if (walls_full(c->d)) (c->ext ? e->full_walls_x : e->full_walls) = true;
         const int flags = (c->d.flag_lMag ? 1 : 0) | (c->d.flag_lRot ? 2 : 0);
         // (a mixed-form member with any branch evaluates every flux in FP64,
         // as alone)
@@ -2036,9 +2040,9 @@ static void ens_enqueue_step(mhd3d_ensemble* e, int p0)
         }
         if (e->mixed) {
             mixed_ens_stage(k, e->waves, e->sched, args, e->d_items, e->nitems, e->grid_int, e->d_walls,
-                            e->nwalls, e->grid_wall, e->stream);
+                            e->nwalls, e->grid_wall, e->full_walls, e->stream);
             ext_ens_stage_s32(k, args, e->d_items_x, e->nitems_x, e->grid_x, e->d_walls_x, e->nwalls_x,
-                              e->grid_wall_x, e->stream);
+                              e->grid_wall_x, e->full_walls_x, e->stream);
         } else {
             ens_stage<double>(e, k, args);
         }

@@ -43,24 +43,27 @@ void mixed_stage(bool mag, bool rot, int stage, const StageArgs& a, hipStream_t 
     else stage_mr<false, false>(stage, a, s, waves, sched, target_blocks);
 }
 
-template <bool MAG, bool ROT>
+template <bool MAG, bool ROT, bool FULL>
 static void wall_mr(int stage, const StageArgs& a, dim3 grid, dim3 block, hipStream_t s)
 {
     if (stage == 1)
-        stage_wall_kernel<float, MAG, ROT, 1><<<grid, block, 0, s>>>(a);
+        stage_wall_kernel<float, MAG, ROT, 1, false, false, FULL><<<grid, block, 0, s>>>(a);
     else if (stage == 2)
-        stage_wall_kernel<float, MAG, ROT, 2><<<grid, block, 0, s>>>(a);
+        stage_wall_kernel<float, MAG, ROT, 2, false, false, FULL><<<grid, block, 0, s>>>(a);
     else
-        stage_wall_kernel<float, MAG, ROT, 3><<<grid, block, 0, s>>>(a);
+        stage_wall_kernel<float, MAG, ROT, 3, false, false, FULL><<<grid, block, 0, s>>>(a);
 }
 
-void mixed_wall(bool mag, bool rot, int stage, const StageArgs& a, dim3 grid, dim3 block,
+void mixed_wall(bool mag, bool rot, int stage, bool full, const StageArgs& a, dim3 grid, dim3 block,
                 hipStream_t s)
 {
-    if (mag && rot) wall_mr<true, true>(stage, a, grid, block, s);
-    else if (mag) wall_mr<true, false>(stage, a, grid, block, s);
-    else if (rot) wall_mr<false, true>(stage, a, grid, block, s);
-    else wall_mr<false, false>(stage, a, grid, block, s);
+    if (!full) {
+        if (mag) wall_mr<true, false, false>(stage, a, grid, block, s);
+        else wall_mr<false, false, false>(stage, a, grid, block, s);
+    } else if (mag && rot) wall_mr<true, true, true>(stage, a, grid, block, s);
+    else if (mag) wall_mr<true, false, true>(stage, a, grid, block, s);
+    else if (rot) wall_mr<false, true, true>(stage, a, grid, block, s);
+    else wall_mr<false, false, true>(stage, a, grid, block, s);
 }
 
 }  // namespace mhd

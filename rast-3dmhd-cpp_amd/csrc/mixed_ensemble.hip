@@ -45,7 +45,7 @@ static void ens_launch(int sched, const StageArgs* args, const WorkItem* items, 
 
 void mixed_ens_stage(int stage, int waves, int sched, const StageArgs* args, const WorkItem* items,
                      int nitems, int grid_int, const WallItem* walls, int nwalls, int grid_wall,
-                     hipStream_t s)
+                     bool full_walls, hipStream_t s)
 {
     if (nitems == 0) {
     } else if (waves == 1) {
@@ -57,11 +57,7 @@ void mixed_ens_stage(int stage, int waves, int sched, const StageArgs* args, con
         else if (stage == 2) ens_launch<2, 2>(sched, args, items, nitems, grid_int, s);
         else ens_launch<3, 2>(sched, args, items, nitems, grid_int, s);
     }
-    const dim3 wblk(64, 4, 1);
-    if (nwalls == 0) {
-    } else if (stage == 1) ensemble_wall_kernel<float, 1><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
-    else if (stage == 2) ensemble_wall_kernel<float, 2><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
-    else ensemble_wall_kernel<float, 3><<<grid_wall, wblk, 0, s>>>(args, walls, nwalls);
+    if (nwalls > 0) launch_ens_walls<float, false, false>(stage, full_walls, grid_wall, args, walls, nwalls, s);
 }
 
 }  // namespace mhd

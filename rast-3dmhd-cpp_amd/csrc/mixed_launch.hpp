@@ -20,8 +20,8 @@ const void* mixed_stream_fn(bool mag, int waves, int sched);
 void mixed_stage(bool mag, bool rot, int stage, const StageArgs& a, hipStream_t s, int waves,
                  int sched, int target_blocks);
 
-// Wall planes of one stage (stage_wall_kernel<float, ...>).
-void mixed_wall(bool mag, bool rot, int stage, const StageArgs& a, dim3 grid, dim3 block,
+// Wall planes of one stage (stage_wall_kernel<float, ...>; full: every flux, see wall_point).
+void mixed_wall(bool mag, bool rot, int stage, bool full, const StageArgs& a, dim3 grid, dim3 block,
                 hipStream_t s);
 
 // Host stub of the ensemble's interior stage-2 kernel of the given variant.
@@ -32,6 +32,6 @@ const void* mixed_ens_stage_fn(int waves, int sched);
 // empty list launches nothing.
 void mixed_ens_stage(int stage, int waves, int sched, const StageArgs* args, const WorkItem* items,
                      int nitems, int grid_int, const WallItem* walls, int nwalls, int grid_wall,
-                     hipStream_t s);
+                     bool full_walls, hipStream_t s);
 
 }  // namespace mhd
