@@ -27,6 +27,7 @@
 #include "kernels_ensemble.hpp"
 #include "mixed_launch.hpp"
 #include "ext_launch.hpp"
+#include "transfer.hpp"
 
 using namespace mhd;
 
@@ -50,8 +51,7 @@ struct mhd3d_ctx {
     CflPart* cfl_parts = nullptr;
     int cfl_parts_cap = 0;
     bool dt_ready = false;          // ds->dt holds TSTEP of the current state
-    double* host_stage = nullptr;   // pinned, one field
-    hipEvent_t slab_ev[4] = {};     // last copy through each slab of host_stage
+    Staging stage;                  // pinned slabs of the host transfers
     hipStream_t stream = nullptr;
     int cur = 0;
     int device = 0;
@@ -441,7 +441,7 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
     if (hipMalloc(&ctx->ds, sizeof(DevScalars)) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(scalars) failed");
     if (hipMemset(ctx->Z, 0, reg) != hipSuccess || hipMemset(ctx->ds, 0, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_EHIP, "hipMemset failed");
-    if (hipHostMalloc(&ctx->host_stage, (size_t)g.fs * sizeof(double)) != hipSuccess ||
+    if (staging_create(ctx->stage, g, ctx->nf) != hipSuccess ||
         hipHostMalloc(&ctx->hs, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_ENOMEM, "hipHostMalloc failed");
     ctx->bytes += (int64_t)((nU64 + 1) * reg + (ctx->mixed ? 2 * reg32 : 0) + nmet * sizeof(double) +
@@ -498,9 +498,7 @@ extern "C" int mhd3d_destroy(mhd3d_ctx* ctx)
     (void)hipFree(ctx->ft);
     (void)hipFree(ctx->relax_buf);
     (void)hipFree(ctx->rs);
-    for (hipEvent_t& ev : ctx->slab_ev)
-        if (ev) (void)hipEventDestroy(ev);
-    if (ctx->host_stage) (void)hipHostFree(ctx->host_stage);
+    staging_destroy(ctx->stage);
     if (ctx->hs) (void)hipHostFree(ctx->hs);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -527,13 +525,6 @@ extern "C" int mhd3d_geometry(const mhd3d_ctx* ctx, int32_t out[4])
 // ---------------------------------------------------------------------------
 // host <-> device field transfer
 
-// A field moves between the host array ([nz][ny][nx], ghosts included) and
-// the device layout ([nz][nPy][pitch]) through the pinned staging buffer in
-// kSlabs slabs of z planes: a team of host threads repacks one slab while
-// the copy of another is in flight, and each slab's event orders the reuse
-// of its part of the buffer.
-constexpr int kSlabs = 4;
-
 // fn(begin, end) over parts of [0, n) on up to 16 host threads (the CPU
 // share of one GPU on a shared host), at least `grain` items a thread.
 template <typename F>
@@ -559,120 +550,6 @@ static void host_parallel(int64_t n, int64_t grain, const F& fn)
     fn((int64_t)0, n / T);
     for (int64_t t = started; t < T; ++t) fn(n * t / T, n * (t + 1) / T);
     for (std::thread& th : team) th.join();
-}
-
-static int slab_events(mhd3d_ctx* ctx)
-{
-    for (hipEvent_t& ev : ctx->slab_ev)
-        if (!ev) HIPCHK(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    return MHD3D_OK;
-}
-
-// Planes [z0, z1) of slab s.
-static void slab_planes(const Geom& g, int s, int& z0, int& z1)
-{
-    const int zs = (g.nz + kSlabs - 1) / kSlabs;
-    z0 = std::min(g.nz, s * zs);
-    z1 = std::min(g.nz, z0 + zs);
-}
-
-// The host array src into the device field dst (interior x, y of every
-// plane; the stream orders the copies, the caller synchronizes it).
-static int upload_field(mhd3d_ctx* ctx, double* dst, const double* src)
-{
-    const Geom& g = ctx->g;
-    const int nx = g.nPx + 2, ny = g.nPy + 2;
-    double* h = ctx->host_stage;
-    int rc = slab_events(ctx);
-    if (rc) return rc;
-    for (int s = 0; s < kSlabs; ++s) {
-        int z0, z1;
-        slab_planes(g, s, z0, z1);
-        if (z0 >= z1) break;
-        HIPCHK(ctx, hipEventSynchronize(ctx->slab_ev[s]));   // the slab's last copy is done
-        host_parallel(z1 - z0, 1, [&](int64_t p0, int64_t p1) {
-            for (int64_t z = z0 + p0; z < z0 + p1; ++z)
-                for (int y = 0; y < g.nPy; ++y) {
-                    double* d = h + (size_t)z * g.plane + (size_t)y * g.pitch;
-                    std::memcpy(d, src + ((size_t)z * ny + (y + 1)) * nx + 1, g.nPx * sizeof(double));
-                    if (g.pitch > g.nPx) std::memset(d + g.nPx, 0, (g.pitch - g.nPx) * sizeof(double));
-                }
-        });
-        const size_t off = (size_t)z0 * g.plane;
-        HIPCHK(ctx, hipMemcpyAsync(dst + off, h + off, (size_t)(z1 - z0) * g.plane * sizeof(double),
-                                   hipMemcpyHostToDevice, ctx->stream));
-        HIPCHK(ctx, hipEventRecord(ctx->slab_ev[s], ctx->stream));
-    }
-    return MHD3D_OK;
-}
-
-// nf device fields from src (field stride fs) into the host arrays dst[f]:
-// the slab copies run ahead of the unpacking by one buffer.  periodic: the
-// x and y ghosts take the periodic copies (3dmhdmpi.h:65-68,118-121,135-142)
-// and every plane is written (the state); otherwise ghosts and the z ghost
-// planes are zero (fluxes).
-static int download_fields(mhd3d_ctx* ctx, double* const* dst, const double* src, int nf, bool periodic)
-{
-    const Geom& g = ctx->g;
-    const int nx = g.nPx + 2, ny = g.nPy + 2;
-    double* h = ctx->host_stage;
-    int rc = slab_events(ctx);
-    if (rc) return rc;
-    int ns = 0;   // slabs with planes
-    for (int s = 0; s < kSlabs; ++s) {
-        int z0, z1;
-        slab_planes(g, s, z0, z1);
-        if (z0 < z1) ns = s + 1;
-    }
-    const int jobs = nf * ns;
-    auto issue = [&](int j) -> int {
-        const int f = j / ns, s = j % ns;
-        int z0, z1;
-        slab_planes(g, s, z0, z1);
-        const size_t off = (size_t)z0 * g.plane;
-        HIPCHK(ctx, hipMemcpyAsync(h + off, src + (size_t)f * g.fs + off, (size_t)(z1 - z0) * g.plane * sizeof(double),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipEventRecord(ctx->slab_ev[s], ctx->stream));
-        return MHD3D_OK;
-    };
-    for (int j = 0; j < std::min(ns, jobs); ++j) {
-        rc = issue(j);
-        if (rc) return rc;
-    }
-    for (int j = 0; j < jobs; ++j) {
-        const int f = j / ns, s = j % ns;
-        int z0, z1;
-        slab_planes(g, s, z0, z1);
-        HIPCHK(ctx, hipEventSynchronize(ctx->slab_ev[s]));
-        double* out = dst[f];
-        host_parallel(z1 - z0, 1, [&](int64_t p0, int64_t p1) {
-            for (int64_t z = z0 + p0; z < z0 + p1; ++z) {
-                double* pl = out + (size_t)z * ny * nx;
-                if (!periodic && (z == 0 || z == g.nz - 1)) {
-                    std::memset(pl, 0, (size_t)ny * nx * sizeof(double));
-                    continue;
-                }
-                for (int y = 0; y < g.nPy; ++y) {
-                    double* row = pl + (size_t)(y + 1) * nx;
-                    std::memcpy(row + 1, h + (size_t)z * g.plane + (size_t)y * g.pitch, g.nPx * sizeof(double));
-                    row[0] = periodic ? row[nx - 2] : 0.0;
-                    row[nx - 1] = periodic ? row[1] : 0.0;
-                }
-                if (periodic) {
-                    std::memcpy(pl, pl + (size_t)(ny - 2) * nx, nx * sizeof(double));
-                    std::memcpy(pl + (size_t)(ny - 1) * nx, pl + (size_t)nx, nx * sizeof(double));
-                } else {
-                    std::memset(pl, 0, nx * sizeof(double));
-                    std::memset(pl + (size_t)(ny - 1) * nx, 0, nx * sizeof(double));
-                }
-            }
-        });
-        if (j + ns < jobs) {
-            rc = issue(j + ns);
-            if (rc) return rc;
-        }
-    }
-    return MHD3D_OK;
 }
 
 // Background of the mixed form from the state being set: RO0(z), TT0(z) (and
@@ -772,13 +649,11 @@ extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
     ctx->dt_ready = false;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
-    for (int f = 0; f < ctx->nf; ++f) {
-        int rc = upload_field(ctx, ctx->U[ctx->cur] + (size_t)f * ctx->g.fs, fields[f]);
-        if (rc) return rc;
-    }
     // the other U buffers need the z ghost planes too (stage kernels never
     // write them)
-    const int64_t n = ctx->g.fs * ctx->nf;
+    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    HIPCHK(ctx, upload_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, fields, ctx->U[ctx->cur],
+                              ctx->mixed ? nullptr : ctx->U[1 - ctx->cur]));
     if (ctx->mixed) {
         int rc = set_background(ctx, fields);
         if (rc) return rc;
@@ -786,9 +661,6 @@ extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
             to_f32_dev_kernel<<<1024, 256, 0, ctx->stream>>>(ctx->U[0], ctx->U32[k], ctx->g, ctx->nf,
                                                             ctx->bg64);
         HIPCHK(ctx, hipGetLastError());
-    } else {
-        HIPCHK(ctx, hipMemcpyAsync(ctx->U[1 - ctx->cur], ctx->U[ctx->cur], (size_t)n * sizeof(double),
-                                   hipMemcpyDeviceToDevice, ctx->stream));
     }
     clear_halt_kernel<<<1, 1, 0, ctx->stream>>>(ctx->ds);   // a new state runs again
     if (ctx->rs) relax_clear_exit_kernel<<<1, 1, 0, ctx->stream>>>(ctx->rs);
@@ -852,7 +724,9 @@ extern "C" int mhd3d_get_state(mhd3d_ctx* ctx, double* const* fields)
     if (!ctx || !fields) return MHD3D_EINVAL;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
-    return download_fields(ctx, fields, ctx->U[ctx->cur], ctx->nf, true);
+    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    HIPCHK(ctx, download_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, ctx->U[ctx->cur], true, fields));
+    return MHD3D_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1337,7 +1211,6 @@ extern "C" int mhd3d_fluxes(mhd3d_ctx* ctx, double* const* flux)
         HIPCHK(ctx, hipMalloc(&ctx->F, reg));
         ctx->bytes += (int64_t)reg;
     }
-    HIPCHK(ctx, hipMemsetAsync(ctx->F, 0, reg, ctx->stream));
     if (ctx->ext_timedep) {
         DevScalars hs;
         HIPCHK(ctx, hipMemcpyAsync(&hs, ctx->ds, sizeof(DevScalars), hipMemcpyDeviceToHost, ctx->stream));
@@ -1360,10 +1233,9 @@ extern "C" int mhd3d_fluxes(mhd3d_ctx* ctx, double* const* flux)
     else if (rot) flux_only_kernel<false, true><<<grd, blk, 0, ctx->stream>>>(a, ctx->F);
     else flux_only_kernel<false, false><<<grd, blk, 0, ctx->stream>>>(a, ctx->F);
     HIPCHK(ctx, hipGetLastError());
-    {
-        int rc = download_fields(ctx, flux, ctx->F, ctx->nf, false);
-        if (rc) return rc;
-    }
+    // (the packing writes zeros for the ghosts, which nothing evaluates)
+    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    HIPCHK(ctx, download_fields(g, ctx->nf, ctx->stage, ctx->stream, ctx->F, false, flux));
     if (ctx->xa.flags & EXT_RLAX) {
         // the reference's fluxes() ends in exit_err at an exit point: the
         // fluxes are complete, then the domain stops
