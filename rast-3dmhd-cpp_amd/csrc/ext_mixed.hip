@@ -40,7 +40,7 @@ void launch_s32(const StageArgs& a, hipStream_t s, int target_blocks)
 {
     const StreamPlan p = stream_plan(a.g, target_blocks);
     stage_stream_kernel<double, MAG, ROT, STAGE, kWavesS32<MAG, STAGE, M>, kOneBarrierS32<MAG, STAGE, M>, true, true, M, true>
-        <<<p.nblocks, dim3(STX, STY, 1), 0, s>>>(a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
+        <<<p.nblocks, dim3(STX, STY, 1), 0, s>>>(a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap, StepEnds{});
 }
 
 template <int M>

@@ -38,7 +38,7 @@ void launch_m(const StageArgs& a, hipStream_t s, int target_blocks)
 {
     const StreamPlan p = stream_plan(a.g, target_blocks);
     stage_stream_kernel<double, MAG, ROT, STAGE, kWaves<MAG, STAGE, M>, kOneBarrier<MAG, STAGE, M>, true, true, M>
-        <<<p.nblocks, dim3(STX, STY, 1), 0, s>>>(a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
+        <<<p.nblocks, dim3(STX, STY, 1), 0, s>>>(a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap, StepEnds{});
 }
 
 template <int M>

@@ -116,6 +116,8 @@ struct DevScalars {
     double dt_min;         // DT guard threshold (0: no guard)
     double nit_call0;      // nIt at the start of the current step call
     double nit_stop;       // stop after this many steps in all (0: no budget)
+    unsigned int arrived;  // blocks of a closing stage-3 launch that are done (0 between launches)
+    unsigned int pad;
 };
 
 // HALT_EXIT: the reference's program exits at this point (RLAX, 3dmhdsub.h:
@@ -418,6 +420,137 @@ __device__ __forceinline__ void cfl_block_reduce(CflAcc& a, CflPart* part, int b
     cfl_block_reduce(a, part, b, sh);
 }
 
+// The DT guard of the reference's driver (3dmhd.cpp:292): after a step whose
+// DT fell below dt_min the run halts -- here every later kernel of the
+// domain returns at once, leaving the state of that step.
+__device__ __forceinline__ void clock_and_guard(DevScalars* s)
+{
+    s->timc += s->dt;
+    s->nit += 1.0;
+    s->dt_last = s->dt;
+    if (s->dt_min > 0.0 && s->dt < s->dt_min) s->halted |= HALT_GUARD;
+    if (s->nit_stop > 0.0 && s->nit >= s->nit_stop) s->halted |= HALT_STOP;
+}
+
+// Reduces the per-block partials in a fixed order (one block of 256 threads:
+// strided per-thread reduction, then the block reduction) and forms
+// DT = SFF * min(...) as 3dmhdsub.h:101-105.  sh: shared memory the caller
+// lends; load(p) reads one record.
+template <typename LD>
+__device__ __forceinline__ void cfl_finalize_block(const CflPart* part, int nparts, DevScalars* s, const Phys& c,
+                                                   int mag, double (*sh)[256], LD load)
+{
+    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+    double w[4] = {1e99, 1e99, 1e99, 1e99};
+    double um = 0.0, bad = 0.0;
+    for (int b = t; b < nparts; b += 256) {
+        const CflPart r = load(part + b);
+        for (int k = 0; k < 4; ++k) w[k] = ref_min(w[k], r.w[k]);
+        um = ref_max(um, r.um);
+        bad = ref_max(bad, r.bad);
+    }
+    for (int k = 0; k < 4; ++k) sh[k][t] = w[k];
+    sh[4][t] = um;
+    sh[5][t] = bad;
+    __syncthreads();
+    for (int st = 128; st > 0; st >>= 1) {
+        if (t < st) {
+            for (int k = 0; k < 4; ++k) sh[k][t] = ref_min(sh[k][t], sh[k][t + st]);
+            sh[4][t] = ref_max(sh[4][t], sh[4][t + st]);
+            sh[5][t] = ref_max(sh[5][t], sh[5][t + st]);
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        for (int k = 0; k < 4; ++k) w[k] = sh[k][0];
+        s->umach = sqrt(sh[4][0]);
+        for (int k = 0; k < 4; ++k) s->wmin[k] = w[k];
+        if (sh[5][0] != 0.0) s->nonfinite = 1u;
+        if (mag)
+            s->dt = c.SFF * ref_min(ref_min(w[0], w[1]), ref_min(w[2], w[3]));
+        else
+            s->dt = c.SFF * ref_min(ref_min(w[0], w[1]), w[2]);
+    }
+}
+
+__device__ __forceinline__ void cfl_finalize_block(const CflPart* __restrict__ part, int nparts,
+                                                   DevScalars* s, const Phys& c, int mag)
+{
+    __shared__ double sh[6][256];
+    cfl_finalize_block(part, nparts, s, c, mag, sh, [](const CflPart* p) { return *p; });
+}
+
+// What the launches of a step do besides at the ends of the step and of a step
+// call: first (stage 1) starts the call's bookkeeping as call_begin_kernel,
+// close (the last launch of stage 3, with nparts TSTEP records in all) closes
+// the step as step_close_kernel, last publishes the scalars to the host's
+// pinned copy `host`.  Launches of their own for these took 13 of 62 us a step
+// call on 32^3.
+struct StepEnds {
+    DevScalars* ds;
+    DevScalars* host;
+    int first, close, last, nparts;
+};
+
+// A TSTEP record that another block of the same launch reads, moved with
+// device-scope accesses: they pass by the caches that are not coherent
+// between XCDs, so no block has to write back its whole L2 (a device-scope
+// release in each of 352 blocks took 20 us of a 53 us launch).
+__device__ __forceinline__ void store_part(CflPart* p, const CflPart& v)
+{
+    const double* s = reinterpret_cast<const double*>(&v);
+    double* d = reinterpret_cast<double*>(p);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(CflPart) / sizeof(double)); ++k)
+        __hip_atomic_store(d + k, s[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ CflPart load_part(const CflPart* p)
+{
+    CflPart v;
+    double* d = reinterpret_cast<double*>(&v);
+    const double* s = reinterpret_cast<const double*>(p);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(CflPart) / sizeof(double)); ++k)
+        d[k] = __hip_atomic_load(s + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+}
+
+// Shared memory step_end_block needs.
+constexpr int STEP_END_LDS = (int)sizeof(double) * 6 * 256 + (int)sizeof(CflPart) + 16;
+
+// End of a stage-3 block of a closing launch of nblocks blocks: its record (in
+// place `slot`), then the count of blocks done; the last one closes the step (clock, DT guard, step budget,
+// the next DT).  Every block of the grid comes here once, none of them waits
+// for another.  lds: STEP_END_LDS bytes no thread uses any more.
+__device__ __forceinline__ void step_end_block(CflAcc& cfl, CflPart* parts, int slot, int nblocks, const StepEnds& e,
+                                               const Phys& c, int mag, char* lds)
+{
+    constexpr int RED = (int)sizeof(double) * 6 * 256;
+    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+    CflPart* rec = reinterpret_cast<CflPart*>(lds + RED);
+    int* last = reinterpret_cast<int*>(lds + RED + sizeof(CflPart));
+    __syncthreads();
+    if (parts) cfl_block_reduce(cfl, rec, 0, reinterpret_cast<double (*)[16]>(lds));   // thread 0 writes rec
+    if (t == 0) {
+        if (parts) store_part(parts + slot, *rec);
+        // the record has reached the device's point of coherence before this block counts as done
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        *last = __hip_atomic_fetch_add(&e.ds->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                (unsigned)nblocks - 1u;
+    }
+    __syncthreads();
+    if (!*last) return;
+    if (t == 0) {
+        e.ds->arrived = 0u;
+        clock_and_guard(e.ds);
+    }
+    __syncthreads();
+    if (parts && !(e.ds->halted & HALT_GUARD))
+        cfl_finalize_block(parts, e.nparts, e.ds, c, mag, reinterpret_cast<double (*)[256]>(lds),
+                           [](const CflPart* q) { return load_part(q); });
+    if (e.last && t == 0) *e.host = *e.ds;   // thread 0 wrote the scalars
+}
+
 // ---------------------------------------------------------------------------
 // Interior planes of one RK stage, one thread per point (baseline form).
 // Stage k: F = fluxes(Uin); Uout = Zin + GAM_k*DT*F; Z = Uout + ZETA_k*DT*F
@@ -635,19 +768,27 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
 // stencils), so the register allocator keeps the occupancy; the off-default
 // variant needs the registers of one wave.
 template <typename T, bool MAG, bool ROT, int STAGE, bool EXT = false, bool S32 = false, bool FULL = true>
-__global__ void __launch_bounds__(256, EXT ? 1 : (sizeof(T) == 4 ? 2 : 3)) stage_wall_kernel(StageArgs a)
+__global__ void __launch_bounds__(256, EXT ? 1 : (sizeof(T) == 4 ? 2 : 3)) stage_wall_kernel(StageArgs a, StepEnds e)
 {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y * blockDim.y + threadIdx.y;
     const bool top = blockIdx.z == 0;
-    if (domain_halted(a)) return;
+    const int b = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (domain_halted(a)) {
+        if (STAGE == 3 && e.last && b == 0 && threadIdx.x == 0 && threadIdx.y == 0) *e.host = *e.ds;
+        return;
+    }
     // every thread reaches the block reduction below; threads outside the
     // domain only contribute the identity
     CflAcc cfl;
     if (x < a.g.nPx && y < a.g.nPy) wall_point<T, MAG, ROT, STAGE, EXT, S32, FULL>(a, x, y, top, cfl);
-    if (STAGE == 3 && a.cfl_parts) {
-        const int b = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-        cfl_block_reduce(cfl, a.cfl_parts, a.cfl_base + b);
+    if constexpr (STAGE == 3) {
+        __shared__ __align__(16) char lds[STEP_END_LDS];
+        if (e.close)
+            step_end_block(cfl, a.cfl_parts, a.cfl_base + b, gridDim.x * gridDim.y * gridDim.z, e, a.c, MAG ? 1 : 0,
+                           lds);
+        else if (a.cfl_parts)
+            cfl_block_reduce(cfl, a.cfl_parts, a.cfl_base + b, reinterpret_cast<double (*)[16]>(lds));
     }
 }
 
@@ -734,57 +875,6 @@ __global__ void __launch_bounds__(256) cfl_kernel(Geom g, Phys c, Metric m,
     }
     const int b = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
     cfl_block_reduce(acc, part, b);
-}
-
-// The DT guard of the reference's driver (3dmhd.cpp:292): after a step whose
-// DT fell below dt_min the run halts -- here every later kernel of the
-// domain returns at once, leaving the state of that step.
-__device__ __forceinline__ void clock_and_guard(DevScalars* s)
-{
-    s->timc += s->dt;
-    s->nit += 1.0;
-    s->dt_last = s->dt;
-    if (s->dt_min > 0.0 && s->dt < s->dt_min) s->halted |= HALT_GUARD;
-    if (s->nit_stop > 0.0 && s->nit >= s->nit_stop) s->halted |= HALT_STOP;
-}
-
-// Reduces the per-block partials in a fixed order (one block of 256 threads:
-// strided per-thread reduction, then the block reduction) and forms
-// DT = SFF * min(...) as 3dmhdsub.h:101-105.
-__device__ __forceinline__ void cfl_finalize_block(const CflPart* __restrict__ part, int nparts,
-                                                   DevScalars* s, const Phys& c, int mag)
-{
-    __shared__ double sh[6][256];
-    double w[4] = {1e99, 1e99, 1e99, 1e99};
-    double um = 0.0, bad = 0.0;
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
-        for (int k = 0; k < 4; ++k) w[k] = ref_min(w[k], part[b].w[k]);
-        um = ref_max(um, part[b].um);
-        bad = ref_max(bad, part[b].bad);
-    }
-    for (int k = 0; k < 4; ++k) sh[k][threadIdx.x] = w[k];
-    sh[4][threadIdx.x] = um;
-    sh[5][threadIdx.x] = bad;
-    __syncthreads();
-    for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) {
-            for (int k = 0; k < 4; ++k)
-                sh[k][threadIdx.x] = ref_min(sh[k][threadIdx.x], sh[k][threadIdx.x + st]);
-            sh[4][threadIdx.x] = ref_max(sh[4][threadIdx.x], sh[4][threadIdx.x + st]);
-            sh[5][threadIdx.x] = ref_max(sh[5][threadIdx.x], sh[5][threadIdx.x + st]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < 4; ++k) w[k] = sh[k][0];
-        s->umach = sqrt(sh[4][0]);
-        for (int k = 0; k < 4; ++k) s->wmin[k] = w[k];
-        if (sh[5][0] != 0.0) s->nonfinite = 1u;
-        if (mag)
-            s->dt = c.SFF * ref_min(ref_min(w[0], w[1]), ref_min(w[2], w[3]));
-        else
-            s->dt = c.SFF * ref_min(ref_min(w[0], w[1]), w[2]);
-    }
 }
 
 MHD_TU_LOCAL __global__ void __launch_bounds__(256) cfl_finalize_kernel(const CflPart* __restrict__ part,

@@ -618,24 +618,57 @@ __device__ __forceinline__ void stage_item(const StageArgs& a, int tile_x, int t
 }
 
 // First plane of z chunk k of nch over the planes 2 .. nPz-1: the chunks hold
-// q = (nPz-2)/nch planes, the first (nPz-2) mod nch of them one more.
+// q = (nPz-2)/nch planes; the (nPz-2) mod nch planes left over go one each to
+// the first chunk, the last one, the second, the third, ...
 __host__ __device__ __forceinline__ int chunk_begin(int nPz, int nch, int q, int k)
 {
-    const int r = nPz - 2 - q * nch;
-    return 2 + k * q + (k < r ? k : r);
+    const int r = nPz - 2 - q * nch, m = r > 1 ? r - 1 : r;
+    return 2 + k * q + (k == nch ? r : (k < m ? k : m));
+}
+
+// The wall points of a tile's columns, after its thread has written their
+// first two planes inward: BCON reads only what this thread wrote.
+template <typename T, bool MAG, int STAGE>
+__device__ __forceinline__ void item_walls(const StageArgs& a, int tile_x, int tile_y, bool top, bool bottom,
+                                           CflAcc& cfl)
+{
+    const int x = tile_x * STX + threadIdx.x, y = tile_y * STY + threadIdx.y;
+    if (x >= a.g.nPx || y >= a.g.nPy) return;
+    if (top) wall_point<T, MAG, false, STAGE, false, false, false>(a, x, y, true, cfl);
+    if (bottom) wall_point<T, MAG, false, STAGE, false, false, false>(a, x, y, false, cfl);
 }
 
 // One stage of one domain: block -> (tile, z chunk) work item.  With
 // xcd_remap, consecutive tiles go to the same XCD (blocks are dealt to the 8
 // XCDs round-robin) so halo re-reads hit its L2.
+// WALLS: the blocks of the first and of the last chunk, which have written
+// the two planes BCON reads, take their columns' wall points as well (the
+// lean ones, see wall_point) and a stage-3 launch closes the step: one launch
+// per stage.  See walls_in_stage for where that pays.  Built for the default
+// variants only (default_variant), which need no accumulation registers; a
+// build of the mixed (1 wave, undeferred) variant that spilled to them
+// flagged finite states as non-finite.
 template <typename T, bool MAG, bool ROT, int STAGE, int WAVES, bool ONE_BARRIER, bool DEFER,
-          bool EXT = false, int EXTM = EXT_INTERIOR, bool S32 = false>
-__global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, int zchunk, int nch,
-                                                                  int ntx, int nty, int xcd_remap)
+          bool EXT = false, int EXTM = EXT_INTERIOR, bool S32 = false, bool WALLS = false>
+__global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, int zchunk, int nch, int ntx, int nty,
+                                                                  int xcd_remap, StepEnds e)
 {
-    __shared__ __align__(16)
-        char lds[StageLds<T, MAG, STAGE, ONE_BARRIER, DEFER, EXT && (EXTM & (EXT_DH | EXT_DV)) != 0>::bytes];
-    if (domain_halted(a)) return;
+    constexpr int NEED =
+        StageLds<T, MAG, STAGE, ONE_BARRIER, DEFER, EXT && (EXTM & (EXT_DH | EXT_DV)) != 0>::bytes;
+    // the FP32 MHD kernels with walls ask for more than a third of a CU's LDS:
+    // the scheduler aims at the occupancy the LDS allows, and would fit stage
+    // 2 into three waves per SIMD with fewer loads in flight (512^2 x 256: 3.16
+    // ms against 2.78)
+    constexpr int LDS = sizeof(T) == 4 && MAG && WALLS && NEED < 55 * 1024 ? 55 * 1024 : NEED;
+    __shared__ __align__(16) char lds[LDS];
+    if (STAGE == 1 && e.first && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
+        e.ds->nonfinite = 0u;
+        e.ds->nit_call0 = e.ds->nit;
+    }
+    if (domain_halted(a)) {
+        if (WALLS && STAGE == 3 && e.last && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *e.host = *e.ds;
+        return;
+    }
     const int nb = gridDim.x;
     const int bid = blockIdx.x;
     const int logical = xcd_remap ? (bid % 8) * (nb / 8) + bid / 8 : bid;
@@ -647,7 +680,11 @@ __global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, i
     const int ze = chunk_begin(a.g.nPz, nch, zchunk, chunk + 1);
     CflAcc cfl;   // stage 3: TSTEP of the next step on the new state
     stage_item<T, MAG, ROT, STAGE, ONE_BARRIER, DEFER, EXT, EXTM, S32>(a, tile_x, tile_y, zb, ze, lds, cfl);
-    if (STAGE == 3 && a.cfl_parts) {
+    if constexpr (WALLS) item_walls<T, MAG, STAGE>(a, tile_x, tile_y, chunk == 0, chunk == nch - 1, cfl);
+    if constexpr (STAGE == 3 && WALLS) {
+        static_assert(LDS >= STEP_END_LDS, "the close of a step borrows the planes");
+        if (e.close) step_end_block(cfl, a.cfl_parts, blockIdx.x, gridDim.x, e, a.c, MAG ? 1 : 0, lds);
+    } else if (STAGE == 3 && a.cfl_parts) {
         // the reduction borrows the plane buffers (a separate 768 B would
         // take an iD variant's two blocks per CU over the CU's LDS)
         __syncthreads();
@@ -655,13 +692,20 @@ __global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, i
     }
 }
 
+// The variants contexts start with (the fastest measured at 256x256x128 and
+// 512x512x256): FP64 MHD one wave, two barriers, deferred; FP64 hydro one
+// wave, one barrier, deferred; mixed two waves, two barriers, deferred.
+constexpr int default_waves(bool mixed) { return mixed ? 2 : 1; }
+constexpr int default_sched(bool mixed, bool mag) { return mixed || mag ? 2 : 3; }
+
 struct StreamPlan {
     int zchunk, nchunks, ntx, nty, nblocks, xcd_remap;
 };
 
 // Work decomposition of one domain: 32 x 8 tiles times the z chunks that make
 // about target_blocks items (at least min_planes planes each), the planes
-// dealt evenly to the chunks.
+// dealt evenly to the chunks; the first and the last chunk hold at least two
+// planes (item_walls).
 inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024, int min_planes = 1)
 {
     StreamPlan p;
@@ -672,6 +716,7 @@ inline StreamPlan stream_plan(const Geom& g, int target_blocks = 1024, int min_p
     int nch = (target_blocks + tiles - 1) / tiles;
     const int maxch = nint / min_planes > 0 ? nint / min_planes : 1;
     if (nch > maxch) nch = maxch;
+    if (nch > nint - 2 && nch > nint / 2) nch = nint - 2;
     if (nch < 1) nch = 1;
     p.zchunk = nint / nch;
     p.nchunks = nch;
@@ -715,50 +760,53 @@ inline int round_blocks(const Geom& g, int resident, int max_planes)
     return tiles * best_n;
 }
 
-// Launch of one interior stage.  sched bit 0: one barrier per plane
-// (ONE_BARRIER), bit 1: deferred update (DEFER); waves: register budget.
-template <typename T, bool MAG, bool ROT, int STAGE, int WAVES>
-static void launch_stream_w(const StageArgs& a, hipStream_t s, const StreamPlan& p, int sched)
+// Launch of one stage.  sched bit 0: one barrier per plane (ONE_BARRIER), bit
+// 1: deferred update (DEFER); waves: register budget; walls (default variants
+// only): the build with the wall points.
+template <typename T, bool MAG, bool ROT, int STAGE, int WAVES, bool ONE_BARRIER, bool DEFER>
+static void launch_stream_v(const StageArgs& a, hipStream_t s, const StreamPlan& p, int walls, const StepEnds& e)
 {
+    constexpr bool MIXED = !std::is_same<T, double>::value;
+    constexpr bool DEFAULT = WAVES == default_waves(MIXED) &&
+                             ((ONE_BARRIER ? 1 : 0) | (DEFER ? 2 : 0)) == default_sched(MIXED, MAG);
     dim3 blk(STX, STY, 1);
+    if (DEFAULT && walls)
+        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, ONE_BARRIER, DEFER, false, EXT_INTERIOR, false, DEFAULT>
+            <<<p.nblocks, blk, 0, s>>>(a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap, e);
+    else
+        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, ONE_BARRIER, DEFER><<<p.nblocks, blk, 0, s>>>(
+            a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap, e);
+}
+
+template <typename T, bool MAG, bool ROT, int STAGE, int WAVES>
+static void launch_stream_w(const StageArgs& a, hipStream_t s, const StreamPlan& p, int sched, int walls,
+                            const StepEnds& e)
+{
     switch (sched & 3) {
-    case 0:
-        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, false, false><<<p.nblocks, blk, 0, s>>>(
-            a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
-        break;
-    case 1:
-        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, true, false><<<p.nblocks, blk, 0, s>>>(
-            a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
-        break;
-    case 2:
-        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, false, true><<<p.nblocks, blk, 0, s>>>(
-            a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
-        break;
-    default:
-        stage_stream_kernel<T, MAG, ROT, STAGE, WAVES, true, true><<<p.nblocks, blk, 0, s>>>(
-            a, p.zchunk, p.nchunks, p.ntx, p.nty, p.xcd_remap);
-        break;
+    case 0: launch_stream_v<T, MAG, ROT, STAGE, WAVES, false, false>(a, s, p, walls, e); break;
+    case 1: launch_stream_v<T, MAG, ROT, STAGE, WAVES, true, false>(a, s, p, walls, e); break;
+    case 2: launch_stream_v<T, MAG, ROT, STAGE, WAVES, false, true>(a, s, p, walls, e); break;
+    default: launch_stream_v<T, MAG, ROT, STAGE, WAVES, true, true>(a, s, p, walls, e); break;
     }
 }
 
-// Kernel function of a variant (stage 2 stands for all stages: they share
-// the resource footprint up to the stage-3 CFL partials).
-template <typename T, bool MAG, bool ROT>
+// Kernel function of a variant.
+template <typename T, bool MAG, bool ROT, int STAGE>
 static const void* stream_fn(int waves, int sched)
 {
     if (waves == 1) {
         switch (sched & 3) {
-        case 0: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 1, false, false>;
-        case 1: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 1, true, false>;
-        case 2: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 1, false, true>;
-        default: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 1, true, true>;
+        case 0: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 1, false, false>;
+        case 1: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 1, true, false>;
+        case 2: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 1, false, true>;
+        default: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 1, true, true>;
         }
     }
     switch (sched & 3) {
-    case 0: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 2, false, false>;
-    case 1: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 2, true, false>;
-    case 2: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 2, false, true>;
-    default: return (const void*)stage_stream_kernel<T, MAG, ROT, 2, 2, true, true>;
+    case 0: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 2, false, false>;
+    case 1: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 2, true, false>;
+    case 2: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 2, false, true>;
+    default: return (const void*)stage_stream_kernel<T, MAG, ROT, STAGE, 2, true, true>;
     }
 }
 
@@ -774,15 +822,28 @@ inline int resident_blocks(const void* fn, int threads)
     return per_cu * ncu;
 }
 
+// The fewest resident blocks among the three stages of a variant, which share
+// one launch plan: planned for a stage 2 that fit three blocks per CU beside
+// stages 1 and 3 at two, the mixed form took 1225 us a step on 256^2 x 128
+// instead of 1130.
+template <typename T, bool MAG, bool ROT>
+static int stream_resident(int waves, int sched)
+{
+    const int r1 = resident_blocks(stream_fn<T, MAG, ROT, 1>(waves, sched), STX * STY);
+    const int r2 = resident_blocks(stream_fn<T, MAG, ROT, 2>(waves, sched), STX * STY);
+    const int r3 = resident_blocks(stream_fn<T, MAG, ROT, 3>(waves, sched), STX * STY);
+    return r1 < r2 ? (r1 < r3 ? r1 : r3) : (r2 < r3 ? r2 : r3);
+}
+
 template <typename T, bool MAG, bool ROT, int STAGE>
 static void launch_stream_stage(const StageArgs& a, hipStream_t s, int waves, int sched,
-                                int target_blocks)
+                                int target_blocks, int walls, const StepEnds& e)
 {
     const StreamPlan p = stream_plan(a.g, target_blocks);
     if (waves == 1)
-        launch_stream_w<T, MAG, ROT, STAGE, 1>(a, s, p, sched);
+        launch_stream_w<T, MAG, ROT, STAGE, 1>(a, s, p, sched, walls, e);
     else
-        launch_stream_w<T, MAG, ROT, STAGE, 2>(a, s, p, sched);
+        launch_stream_w<T, MAG, ROT, STAGE, 2>(a, s, p, sched, walls, e);
 }
 
 }  // namespace mhd

@@ -61,8 +61,9 @@ struct mhd3d_ctx {
     // schedule bits (1: one barrier per plane, 2: deferred RK update).
     // Defaults: the fastest variants measured on MI355X at 256x256x128 and
     // 512x512x256 (launches sized to the resident block count).
-    int tune_waves[2][2] = {{1, 1}, {2, 2}};
-    int tune_sched[2][2] = {{3, 2}, {2, 2}};
+    int tune_waves[2][2] = {{default_waves(false), default_waves(false)}, {default_waves(true), default_waves(true)}};
+    int tune_sched[2][2] = {{default_sched(false, false), default_sched(false, true)},
+                            {default_sched(true, false), default_sched(true, true)}};
     bool fuse_cfl = true;           // TSTEP evaluated inside the stage-3 launch
     // off-default branches (iD, lRem, lShr, iTCon 2, TP plume, RLAX): FP64, evaluated
     // by the point and wall kernels
@@ -80,6 +81,8 @@ struct mhd3d_ctx {
     int relax_exit_code = 0;        // RelaxState::exited as last read
     int target_blocks = 0;          // work items of one streaming launch (z chunking);
                                     // 0: the resident blocks of the kernel variant
+    bool ends = false;              // the launches of a step start the call and close the step (StepEnds)
+    bool fold = false;              // a stage is one launch, walls included (walls_in_stage)
     int64_t bytes = 0;
     std::string err;
     // timing
@@ -169,6 +172,9 @@ static int validate(const mhd3d_desc* d, std::string& why)
     if (d->precision != MHD3D_FP64 && d->precision != MHD3D_MIXED) { why = "invalid precision"; return MHD3D_EINVAL; }
     return MHD3D_OK;
 }
+
+// Whether a wall flux other than those of RO, BX, BY has a reader (wall_point).
+static bool walls_full(const mhd3d_desc& d) { return d.flag_iTCon == 3 || d.flag_lShr; }
 
 static Phys make_phys(const mhd3d_desc* d)
 {
@@ -338,16 +344,33 @@ static int setup_ext(mhd3d_ctx* ctx, const mhd3d_desc* d)
 static int variant_resident(const mhd3d_ctx* ctx, int w, int sc)
 {
     const bool mag = ctx->d.flag_lMag != 0;
-    const void* fn;
     if (ctx->mixed && ctx->ext)
-        fn = ext_stream_fn_s32(mag, ext_variant(ctx->xa.flags));
-    else if (ctx->mixed)
-        fn = mixed_stream_fn(mag, w, sc);
-    else if (ext_variant(ctx->xa.flags) != EXTV_NONE)
-        fn = ext_stream_fn(mag, ext_variant(ctx->xa.flags));
-    else
-        fn = mag ? stream_fn<double, true, true>(w, sc) : stream_fn<double, false, true>(w, sc);
-    return resident_blocks(fn, STX * STY);
+        return resident_blocks(ext_stream_fn_s32(mag, ext_variant(ctx->xa.flags)), STX * STY);
+    if (ctx->mixed) return mixed_stream_resident(mag, w, sc);
+    if (ext_variant(ctx->xa.flags) != EXTV_NONE)
+        return resident_blocks(ext_stream_fn(mag, ext_variant(ctx->xa.flags)), STX * STY);
+    return mag ? stream_resident<double, true, true>(w, sc) : stream_resident<double, false, true>(w, sc);
+}
+
+// Whether the blocks of the first and the last z chunk take the walls of
+// their columns in the stage launch.  Where the launch is one round of the
+// resident blocks, a wall launch after it is idle time (FP64, us a step, walls
+// apart -> in the stage: hydro 32^3 47 -> 37, MHD 64^3 85 -> 70, 96x96x64 141
+// -> 132, 256x256x128 1235 -> 1216); with more rounds the first and last
+// chunks' longer blocks cost more than the launch (192x192x96 602 -> 612,
+// 512x512x256 10057 -> 10211).  The mixed form's wall code slows its
+// stages (128x128x64 179 -> 181, 512x512x256 8.67 -> 8.84 ms), so there only
+// for chunks of a few planes (64^3 80 -> 74).
+static bool walls_in_stage(const mhd3d_ctx* ctx, int resident)
+{
+    if (!ctx->ends || walls_full(ctx->d)) return false;
+    const int fm = ctx->mixed ? 1 : 0, ph = ctx->d.flag_lMag ? 1 : 0;
+    if (ctx->tune_waves[fm][ph] != default_waves(ctx->mixed) ||
+        ctx->tune_sched[fm][ph] != default_sched(ctx->mixed, ph != 0))
+        return false;   // the wall code is built into the default variants
+    const StreamPlan p = stream_plan(ctx->g, ctx->target_blocks);
+    if (p.nblocks > resident) return false;
+    return !ctx->mixed || p.zchunk < 4;
 }
 
 extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
@@ -466,13 +489,15 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
     const char* fc = std::getenv("MHD3D_FUSE_CFL");
     if (fc && std::atoi(fc) == 0) ctx->fuse_cfl = false;
     if (ctx->mixed) ctx->kernel_mode = 0;   // the mixed form has only the streaming kernel
-    if (ctx->target_blocks == 0) {
+    {
         const int fm = ctx->mixed ? 1 : 0, ph = desc->flag_lMag ? 1 : 0;
+        const int res = variant_resident(ctx, ctx->tune_waves[fm][ph], ctx->tune_sched[fm][ph]);
         // FP64: z chunks of at most 64 planes (MI355X, FP64 MHD 512x512x256
         // stage kernel: one chunk 3.47 ms, two 3.40, four 3.35, eight 3.74);
         // the mixed form is best with the longest chunks its rounds allow
-        ctx->target_blocks = round_blocks(g, variant_resident(ctx, ctx->tune_waves[fm][ph], ctx->tune_sched[fm][ph]),
-                                          ctx->mixed ? 0 : 64);
+        if (ctx->target_blocks == 0) ctx->target_blocks = round_blocks(g, res, ctx->mixed ? 0 : 64);
+        ctx->ends = !ctx->ext && ctx->kernel_mode == 0;
+        ctx->fold = walls_in_stage(ctx, res);
     }
     *out = ctx;
     return MHD3D_OK;
@@ -771,8 +796,9 @@ static hipEvent_t next_event(mhd3d_ctx* ctx)
 }
 
 template <bool MAG, bool ROT, int STAGE>
-static void launch_stage_t(mhd3d_ctx* ctx, const StageArgs& a)
+static void launch_stage_t(mhd3d_ctx* ctx, const StageArgs& a, const StepEnds& e)
 {
+    const int walls = ctx->fold ? 1 : 0;
     const Geom& g = ctx->g;
     dim3 blk(64, 4, 1);
     const int fm = ctx->mixed ? 1 : 0, ph = MAG ? 1 : 0;
@@ -780,7 +806,7 @@ static void launch_stage_t(mhd3d_ctx* ctx, const StageArgs& a)
         ext_stage_s32(MAG, ROT, STAGE, ext_variant(ctx->xa.flags), a, ctx->stream, ctx->target_blocks);
     } else if (ctx->mixed) {
         mixed_stage(MAG, ROT, STAGE, a, ctx->stream, ctx->tune_waves[fm][ph], ctx->tune_sched[fm][ph],
-                    ctx->target_blocks);
+                    ctx->target_blocks, walls, e);
     } else if (ctx->kernel_mode == 0 && ext_variant(ctx->xa.flags) != EXTV_NONE) {
         ext_stage(MAG, ROT, STAGE, ext_variant(ctx->xa.flags), a, ctx->stream, ctx->target_blocks);
     } else if (ctx->kernel_mode == 1) {
@@ -791,47 +817,47 @@ static void launch_stage_t(mhd3d_ctx* ctx, const StageArgs& a)
             stage_point_kernel<MAG, ROT, STAGE><<<grd, blk, 0, ctx->stream>>>(a);
     } else {
         launch_stream_stage<double, MAG, ROT, STAGE>(a, ctx->stream, ctx->tune_waves[fm][ph],
-                                                     ctx->tune_sched[fm][ph], ctx->target_blocks);
+                                                     ctx->tune_sched[fm][ph], ctx->target_blocks, walls, e);
     }
 }
 
-// Whether a wall flux other than those of RO, BX, BY has a reader (wall_point).
-static bool walls_full(const mhd3d_desc& d) { return d.flag_iTCon == 3 || d.flag_lShr; }
-
 template <bool MAG, bool ROT, int STAGE, bool FULL>
-static void launch_wall_t(mhd3d_ctx* ctx, const StageArgs& a)
+static void launch_wall_t(mhd3d_ctx* ctx, const StageArgs& a, const StepEnds& e)
 {
     const Geom& g = ctx->g;
     dim3 blk(64, 4, 1);
     dim3 grd((g.nPx + 63) / 64, (g.nPy + 3) / 4, 2);
     if (ctx->mixed && ctx->ext)
-        stage_wall_kernel<double, MAG, ROT, STAGE, true, true, FULL><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, true, true, FULL><<<grd, blk, 0, ctx->stream>>>(a, e);
     else if (ctx->mixed)
-        mixed_wall(MAG, ROT, STAGE, FULL, a, grd, blk, ctx->stream);
+        mixed_wall(MAG, ROT, STAGE, FULL, a, e, grd, blk, ctx->stream);
     else if (ctx->ext)
-        stage_wall_kernel<double, MAG, ROT, STAGE, true, false, FULL><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, true, false, FULL><<<grd, blk, 0, ctx->stream>>>(a, e);
     else
-        stage_wall_kernel<double, MAG, ROT, STAGE, false, false, FULL><<<grd, blk, 0, ctx->stream>>>(a);
+        stage_wall_kernel<double, MAG, ROT, STAGE, false, false, FULL><<<grd, blk, 0, ctx->stream>>>(a, e);
 }
 
 template <int STAGE>
-static void launch_stage_k(mhd3d_ctx* ctx, const StageArgs& a, bool wall)
+static void launch_stage_k(mhd3d_ctx* ctx, const StageArgs& a, const StepEnds& e)
 {
     const bool mag = ctx->d.flag_lMag, rot = ctx->d.flag_lRot;
-    if (!wall) {
-        if (mag && rot) launch_stage_t<true, true, STAGE>(ctx, a);
-        else if (mag) launch_stage_t<true, false, STAGE>(ctx, a);
-        else if (rot) launch_stage_t<false, true, STAGE>(ctx, a);
-        else launch_stage_t<false, false, STAGE>(ctx, a);
-    } else {
-        if (!walls_full(ctx->d)) {   // no rotation term in the fluxes kept
-            if (mag) launch_wall_t<true, false, STAGE, false>(ctx, a);
-            else launch_wall_t<false, false, STAGE, false>(ctx, a);
-        } else if (mag && rot) launch_wall_t<true, true, STAGE, true>(ctx, a);
-        else if (mag) launch_wall_t<true, false, STAGE, true>(ctx, a);
-        else if (rot) launch_wall_t<false, true, STAGE, true>(ctx, a);
-        else launch_wall_t<false, false, STAGE, true>(ctx, a);
-    }
+    if (mag && rot) launch_stage_t<true, true, STAGE>(ctx, a, e);
+    else if (mag) launch_stage_t<true, false, STAGE>(ctx, a, e);
+    else if (rot) launch_stage_t<false, true, STAGE>(ctx, a, e);
+    else launch_stage_t<false, false, STAGE>(ctx, a, e);
+}
+
+template <int STAGE>
+static void launch_wall_k(mhd3d_ctx* ctx, const StageArgs& a, const StepEnds& e)
+{
+    const bool mag = ctx->d.flag_lMag, rot = ctx->d.flag_lRot;
+    if (!walls_full(ctx->d)) {   // no rotation term in the fluxes kept
+        if (mag) launch_wall_t<true, false, STAGE, false>(ctx, a, e);
+        else launch_wall_t<false, false, STAGE, false>(ctx, a, e);
+    } else if (mag && rot) launch_wall_t<true, true, STAGE, true>(ctx, a, e);
+    else if (mag) launch_wall_t<true, false, STAGE, true>(ctx, a, e);
+    else if (rot) launch_wall_t<false, true, STAGE, true>(ctx, a, e);
+    else launch_wall_t<false, false, STAGE, true>(ctx, a, e);
 }
 
 // Number of CFL partial records the fused stage-3 launch writes: one per
@@ -843,7 +869,7 @@ static void cfl_part_layout(const mhd3d_ctx* ctx, int& nstream, int& nwall)
         nstream = ((g.nPx + 63) / 64) * ((g.nPy + 3) / 4) * (g.nPz - 2);
     else
         nstream = stream_plan(g, ctx->target_blocks).nblocks;
-    nwall = ((g.nPx + 63) / 64) * ((g.nPy + 3) / 4) * 2;
+    nwall = ctx->fold ? 0 : ((g.nPx + 63) / 64) * ((g.nPy + 3) / 4) * 2;
 }
 
 static int ensure_cfl_parts(mhd3d_ctx* ctx, int n)
@@ -922,7 +948,8 @@ static int run_prepass(mhd3d_ctx* ctx, const StageArgs& a, int k, hipStream_t st
     return run_prepass_t<double>(ctx, a.Uin, k, stream);
 }
 
-static int run_stage(mhd3d_ctx* ctx, int k, bool fused_cfl = false)
+// ends: what the stage's launches do besides.
+static int run_stage(mhd3d_ctx* ctx, int k, bool fused_cfl = false, const StepEnds& ends = StepEnds{})
 {
     StageArgs a = stage_args(ctx, k);
     if (ctx->ext) {
@@ -943,18 +970,22 @@ static int run_stage(mhd3d_ctx* ctx, int k, bool fused_cfl = false)
         if (!e0 || !e1) return fail(ctx, MHD3D_EHIP, "hipEventCreate failed");
         HIPCHK(ctx, hipEventRecord(e0, ctx->stream));
     }
-    if (k == 1) launch_stage_k<1>(ctx, a, false);
-    else if (k == 2) launch_stage_k<2>(ctx, a, false);
-    else launch_stage_k<3>(ctx, a, false);
+    int ns, nw;
+    cfl_part_layout(ctx, ns, nw);
+    // the close belongs to the stage's last launch
+    StepEnds es = ends, ew = ends;
+    es.nparts = ew.nparts = ns + nw;
+    if (!ctx->fold) es.close = es.last = 0;
+    if (k == 1) launch_stage_k<1>(ctx, a, es);
+    else if (k == 2) launch_stage_k<2>(ctx, a, es);
+    else launch_stage_k<3>(ctx, a, es);
     if (ctx->timing) HIPCHK(ctx, hipEventRecord(e1, ctx->stream));
-    if (a.cfl_parts) {
-        int ns, nw;
-        cfl_part_layout(ctx, ns, nw);
-        a.cfl_base = ns;
+    if (!ctx->fold) {
+        if (a.cfl_parts) a.cfl_base = ns;
+        if (k == 1) launch_wall_k<1>(ctx, a, ew);
+        else if (k == 2) launch_wall_k<2>(ctx, a, ew);
+        else launch_wall_k<3>(ctx, a, ew);
     }
-    if (k == 1) launch_stage_k<1>(ctx, a, true);
-    else if (k == 2) launch_stage_k<2>(ctx, a, true);
-    else launch_stage_k<3>(ctx, a, true);
     HIPCHK(ctx, hipGetLastError());
     if (!ctx->mixed) ctx->cur = 1 - ctx->cur;
     return MHD3D_OK;
@@ -1014,7 +1045,10 @@ static int step_core(mhd3d_ctx* ctx, int nsteps, int fixed_dt, double* dt_inout)
     if (!ctx || nsteps < 0) return MHD3D_EINVAL;
     if (fixed_dt && !dt_inout) return fail(ctx, MHD3D_EINVAL, "fixed_dt needs *dt_inout");
     const int cur0 = ctx->cur;
-    call_begin_kernel<<<1, 1, 0, ctx->stream>>>(ctx->ds);
+    // the call's bookkeeping: inside the first stage, unless a TSTEP pass,
+    // which may set the non-finite flag, comes first
+    const bool begin_in_stage = ctx->ends && nsteps > 0 && (fixed_dt || ctx->dt_ready);
+    if (!begin_in_stage) call_begin_kernel<<<1, 1, 0, ctx->stream>>>(ctx->ds);
     if (fixed_dt) {
         set_dt_kernel<<<1, 1, 0, ctx->stream>>>(ctx->ds, *dt_inout);
         HIPCHK(ctx, hipGetLastError());
@@ -1037,10 +1071,18 @@ static int step_core(mhd3d_ctx* ctx, int nsteps, int fixed_dt, double* dt_inout)
             if (rc) return rc;
         }
         for (int k = 1; k <= 3; ++k) {
-            int rc = run_stage(ctx, k, fuse);
+            StepEnds e{ctx->ds, ctx->hs, 0, 0, 0, 0};
+            if (ctx->ends) {
+                e.first = begin_in_stage && k == 1 && n == 0;
+                e.close = k == 3;
+                e.last = k == 3 && n == nsteps - 1 && fuse;
+            }
+            int rc = run_stage(ctx, k, fuse, e);
             if (rc) return rc;
         }
-        if (fuse) {
+        if (ctx->ends) {
+            // closed by its last launch
+        } else if (fuse) {
             int ns, nw;
             cfl_part_layout(ctx, ns, nw);
             step_close_kernel<<<1, 256, 0, ctx->stream>>>(ctx->cfl_parts, ns + nw, ctx->ds, ctx->c,
@@ -1064,7 +1106,9 @@ static int step_core(mhd3d_ctx* ctx, int nsteps, int fixed_dt, double* dt_inout)
         nonfinite_kernel<<<grd, blk, 0, ctx->stream>>>(g, ctx->nf, ctx->U[ctx->cur], ctx->ds);
         HIPCHK(ctx, hipGetLastError());
     }
-    HIPCHK(ctx, hipMemcpyAsync(ctx->hs, ctx->ds, sizeof(DevScalars), hipMemcpyDeviceToHost, ctx->stream));
+    // (a launch that closes the last step has written the host's copy itself)
+    if (!(ctx->ends && fuse && nsteps > 0))
+        HIPCHK(ctx, hipMemcpyAsync(ctx->hs, ctx->ds, sizeof(DevScalars), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     const DevScalars hs = *ctx->hs;
     // the register holding the state: each step taken flips it (three
@@ -1317,6 +1361,7 @@ extern "C" int mhd3d_autotune(mhd3d_ctx* ctx, int steps, double* report, int* nc
     const bool ready_save = ctx->dt_ready;
     const int fm = ctx->mixed ? 1 : 0, ph = ctx->d.flag_lMag ? 1 : 0;
     int best_w = ctx->tune_waves[fm][ph], best_s = ctx->tune_sched[fm][ph], best_t = ctx->target_blocks;
+    bool best_fold = ctx->fold;
     int rc = MHD3D_OK;
     if (hipMemcpyAsync(snap, ctx->U[ctx->cur], reg, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess ||
         hipMemcpyAsync(ds_snap, ctx->ds, sizeof(DevScalars), hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
@@ -1341,7 +1386,9 @@ extern "C" int mhd3d_autotune(mhd3d_ctx* ctx, int steps, double* report, int* nc
             for (int ip = 0; ip < 3 && !rc; ++ip) {
                 ctx->tune_waves[fm][ph] = wv[iw];
                 ctx->tune_sched[fm][ph] = is;
-                ctx->target_blocks = round_blocks(ctx->g, variant_resident(ctx, wv[iw], is), planes[ip]);
+                const int res = variant_resident(ctx, wv[iw], is);
+                ctx->target_blocks = round_blocks(ctx->g, res, planes[ip]);
+                ctx->fold = walls_in_stage(ctx, res);
                 ctx->dt_ready = false;   // the partial records follow the launch size
                 double dt = 0.0;
                 int r = step_core(ctx, 1, 0, &dt);   // warm-up
@@ -1370,6 +1417,7 @@ extern "C" int mhd3d_autotune(mhd3d_ctx* ctx, int steps, double* report, int* nc
                     best_w = wv[iw];
                     best_s = is;
                     best_t = ctx->target_blocks;
+                    best_fold = ctx->fold;
                 }
                 const int rr = restore();
                 if (!rc) rc = rr;
@@ -1379,6 +1427,7 @@ extern "C" int mhd3d_autotune(mhd3d_ctx* ctx, int steps, double* report, int* nc
     ctx->tune_waves[fm][ph] = best_w;
     ctx->tune_sched[fm][ph] = best_s;
     ctx->target_blocks = best_t;
+    ctx->fold = best_fold;
     ctx->dt_ready = false;
     (void)hipFree(snap);
     (void)hipFree(ds_snap);

@@ -12,17 +12,16 @@
 
 namespace mhd {
 
-// Host stub of the interior stage-2 kernel of the given variant (MHD or
-// hydro, with rotation), for occupancy queries.
-const void* mixed_stream_fn(bool mag, int waves, int sched);
+// Resident blocks of a variant (stream_resident; MHD or hydro, with rotation).
+int mixed_stream_resident(bool mag, int waves, int sched);
 
-// Interior planes of one stage (launch_stream_stage<float, ...>).
+// One stage (launch_stream_stage<float, ...>).
 void mixed_stage(bool mag, bool rot, int stage, const StageArgs& a, hipStream_t s, int waves,
-                 int sched, int target_blocks);
+                 int sched, int target_blocks, int walls, const StepEnds& e);
 
 // Wall planes of one stage (stage_wall_kernel<float, ...>; full: every flux, see wall_point).
-void mixed_wall(bool mag, bool rot, int stage, bool full, const StageArgs& a, dim3 grid, dim3 block,
-                hipStream_t s);
+void mixed_wall(bool mag, bool rot, int stage, bool full, const StageArgs& a, const StepEnds& e, dim3 grid,
+                dim3 block, hipStream_t s);
 
 // Host stub of the ensemble's interior stage-2 kernel of the given variant.
 const void* mixed_ens_stage_fn(int waves, int sched);
