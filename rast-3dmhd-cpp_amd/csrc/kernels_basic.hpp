@@ -1060,7 +1060,7 @@ __device__ __forceinline__ double tree_plane_sum(const Geom& g, V value, double*
 }
 
 // The sequential sum of ordered_plane_sum -- the same double, bit for bit --
-// by a block of PW_T threads.  While the running sum s stays inside one
+// by a block of PW_T walker threads.  While the running sum s stays inside one
 // binade, |s| in (2^e, 2^(e+1)), every value it takes is a multiple of that
 // binade's grid u = 2^(e-52): s = M*u with the integer M in (2^52, 2^53).
 // Adding v then gives M' = M + RNE(v/u) (the exact sum's nearest grid
@@ -1088,14 +1088,20 @@ __device__ __forceinline__ double tree_plane_sum(const Geom& g, V value, double*
 //
 // The plane streams through LDS as chunks of PW_C summands in a ring of
 // PW_SLOTS chunks: at a round starting in chunk a, chunks a .. a+2 are
-// resident; the round loads chunk a+3 into registers first and stores it
-// after its own work, in the slot of chunk a-1.  The chunk after the
+// resident; meanwhile PW_T producer threads of the same block (their own
+// waves, at the same barriers) load chunk a+3 and store it after the round in
+// the slot of chunk a-1, so that its addresses and loads are not in the
+// walkers' path.  us a step of iD with lRem, FP64 hydro: 192x192x96 646 ->
+// 626 (a launch 62 -> 56), 256x256x128 1250 -> 1236, 512x512x256 9440 -> 9240;
+// held to 128 VGPRs, as a plane count beyond the CUs needs two blocks on one
+// (256x256x128 with 130: 1377).  The chunk after the
 // plane's last is stored as zeros, summands that add nothing, so a round
 // reads its PW_C summands unchecked.  Ring index r of summand f is
 // f mod PW_RING, stored at r + r/8 so that the threads' strided reads of 8
 // consecutive summands hit distinct banks.  value(y, x) forms the summand of
 // interior point (x, y); the sum is returned to every thread.
-constexpr int PW_T = 256;
+constexpr int PW_T = 256;              // walker threads
+constexpr int PW_B = 2 * PW_T;         // and as many producers
 constexpr int PW_W = PW_T / 64;
 constexpr int PW_R = 8;
 constexpr int PW_C = PW_T * PW_R;
@@ -1169,11 +1175,12 @@ __device__ __forceinline__ double pw_chain(const double* ring, double s, int64_t
 template <typename V>
 __device__ __forceinline__ double walk_plane_sum(const Geom& g, V value, PwShared& sh)
 {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const bool producer = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >= PW_T;   // whole waves
+    const int t = threadIdx.x & (PW_T - 1), lane = t & 63, w = t >> 6;
     const int nPx = g.nPx;
     const int64_t N = (int64_t)nPx * g.nPy;
     const int64_t nch = (N + PW_C - 1) / PW_C;
-    // (y, x) of this thread's summand in the next chunk to load: steps of
+    // producers: (y, x) of this thread's summand in the next chunk to load: steps of
     // PW_T summands within a chunk, PW_C from one chunk to the next
     const int qy = PW_T / nPx, qx = PW_T - qy * nPx;
     const int cy = PW_C / nPx, cx = PW_C - cy * nPx;
@@ -1208,9 +1215,11 @@ __device__ __forceinline__ double walk_plane_sum(const Geom& g, V value, PwShare
 #pragma unroll
         for (int j = 0; j < PW_R; ++j) sh.ring[pw_slot(c * PW_C + t + j * PW_T)] = z ? 0.0 : pre[j];
     };
-    for (int c = 0; c < 3; ++c) {
-        if (c < nch) load_next();
-        store_chunk(c);
+    if (producer) {
+        for (int c = 0; c < 3; ++c) {
+            if (c < nch) load_next();
+            store_chunk(c);
+        }
     }
     int64_t hi = 2;   // highest chunk stored in the ring
     __syncthreads();
@@ -1222,7 +1231,7 @@ __device__ __forceinline__ double walk_plane_sum(const Geom& g, V value, PwShare
     while (p < N) {
         const int64_t a = p / PW_C;
         const bool fetch = hi == a + 2 && a + 3 <= nch;
-        if (fetch && a + 3 < nch) load_next();
+        if (producer && fetch && a + 3 < nch) load_next();
         const double as = fabs(s);
         if (!(as >= 0x1p-1021 && as < __builtin_inf()) || breaks >= budget) {
             const int64_t end = (a + 1) * PW_C < N ? (a + 1) * PW_C : N;
@@ -1239,125 +1248,138 @@ __device__ __forceinline__ double walk_plane_sum(const Geom& g, V value, PwShare
             // accepted prefixes P: M + P in (2^52, 2^53), or its negative
             const double plo = s > 0.0 ? 0x1p52 - M : -0x1p53 - M;
             const double phi = s > 0.0 ? 0x1p53 - M : -0x1p52 - M;
-            const int64_t f0 = p + (int64_t)t * PW_R;
-            double v[PW_R], q[PW_R];
-            unsigned flag = 0;       // summands rejected
-            unsigned halfm = 0;      // halfway cases
-            double acc = 0.0;
+            double T = 0.0;   // the round's whole increment
+            if (producer) {
+                __syncthreads();   // the walkers' totals and parity maps
+                int pin = pw_odd(M);
 #pragma unroll
-            for (int i = 0; i < PW_R; ++i) {
-                v[i] = sh.ring[pw_slot(f0 + i)];
-                const double sc = ldexp(v[i], 52 - e);
-                const double r = rint(sc);
-                const bool half = fabs(sc - r) == 0.5;
-                if (!(fabs(v[i]) < lim)) flag |= 1u << i;
-                if (half) halfm |= 1u << i;
-                acc += half ? sc - 0.5 : r;   // the floor for a halfway case
-                q[i] = acc;
-            }
-            // The parity of the running integer M flips by the parity of a sum
-            // of increments, so a thread without halfway cases passes on its
-            // incoming parity flipped by that of its total.  With them (rare
-            // but for planes of equal or dyadic values): the first one's
-            // rounding bit is the incoming parity ^ g2, added as bf once the
-            // parity is known; it leaves M even, so each later one's bit is
-            // the parity of the increments since the tie before it, and the
-            // parity passed on is that of the increments after the last tie.
-            const bool seen = halfm != 0;
-            unsigned after = 0;      // summands from the first halfway case on
-            int g2 = 0, gam;
-            if (!seen) {
-                gam = pw_odd(acc);
+                for (int ww = 0; ww < PW_W; ++ww) {
+                    T += pin ? sh.tot[1][ww] : sh.tot[0][ww];
+                    const unsigned pm = sh.par[ww];
+                    pin = (pm & 1u) ? (pin ^ (int)(pm >> 1)) : (int)(pm >> 1);
+                }
+                __syncthreads();   // the first rejected summand
             } else {
-                const int fh = __builtin_ctz(halfm);
-                after = ~0u << fh;
-                double q0L = 0.0, add = 0.0;   // the prefix at the last tie; later rounding bits
+                const int64_t f0 = p + (int64_t)t * PW_R;
+                double v[PW_R], q[PW_R];
+                unsigned flag = 0;       // summands rejected
+                unsigned halfm = 0;      // halfway cases
+                double acc = 0.0;
 #pragma unroll
                 for (int i = 0; i < PW_R; ++i) {
-                    const double q0 = q[i];
-                    if (i == fh) {
-                        g2 = pw_odd(q0);
-                        q0L = q0;
-                    } else if (i > fh && ((halfm >> i) & 1u)) {
-                        add += (double)pw_odd(q0 - q0L);
-                        q0L = q0;
-                    }
-                    q[i] = q0 + add;
+                    v[i] = sh.ring[pw_slot(f0 + i)];
+                    const double sc = ldexp(v[i], 52 - e);
+                    const double r = rint(sc);
+                    const bool half = fabs(sc - r) == 0.5;
+                    if (!(fabs(v[i]) < lim)) flag |= 1u << i;
+                    if (half) halfm |= 1u << i;
+                    acc += half ? sc - 0.5 : r;   // the floor for a halfway case
+                    q[i] = acc;
                 }
-                gam = pw_odd(acc - q0L);
-                acc = q[PW_R - 1];
-            }
-            // incoming parity of this lane: base ^ (dep & the wave's incoming parity)
-            const uint64_t Rm = __ballot(seen);
-            const uint64_t Xb = __ballot(gam);
-            const uint64_t Rb = Rm & below;
-            int base, dep;
-            if (Rb) {
-                const int r = 63 - __clzll((long long)Rb);
-                base = __popcll(Xb & below & ~((uint64_t(1) << r) - 1)) & 1;
-                dep = 0;
-            } else {
-                base = __popcll(Xb & below) & 1;
-                dep = 1;
-            }
-            const int b0 = base ^ g2;   // the first halfway case's bit for an incoming parity 0
-            double incl;
-            double E = pw_wave_scan(acc + (seen ? (double)b0 : 0.0), incl);
-            // for an incoming parity 1 the lanes with seen && dep add 1 - 2*b0 instead of b0
-            // (counts as signed ints: __popcll is unsigned)
-            const uint64_t up1 = __ballot(seen && dep && !b0), dn1 = __ballot(seen && dep && b0);
-            if (lane == 63) {
-                sh.tot[0][w] = incl;
-                sh.tot[1][w] = incl + (double)((int)__popcll(up1) - (int)__popcll(dn1));
-            }
-            if (lane == 0) {
-                int xw;
-                if (Rm) {
-                    const int r = 63 - __clzll((long long)Rm);
-                    xw = __popcll(Xb & ~((uint64_t(1) << r) - 1)) & 1;
+                // The parity of the running integer M flips by the parity of a sum
+                // of increments, so a thread without halfway cases passes on its
+                // incoming parity flipped by that of its total.  With them (rare
+                // but for planes of equal or dyadic values): the first one's
+                // rounding bit is the incoming parity ^ g2, added as bf once the
+                // parity is known; it leaves M even, so each later one's bit is
+                // the parity of the increments since the tie before it, and the
+                // parity passed on is that of the increments after the last tie.
+                const bool seen = halfm != 0;
+                unsigned after = 0;      // summands from the first halfway case on
+                int g2 = 0, gam;
+                if (!seen) {
+                    gam = pw_odd(acc);
                 } else {
-                    xw = __popcll(Xb) & 1;
-                }
-                sh.par[w] = (Rm ? 0u : 1u) | ((unsigned)xw << 1);
-            }
-            __syncthreads();
-            int pin = pw_odd(M), mine = 0;
-            double Ew = 0.0, T = 0.0;
-#pragma unroll
-            for (int ww = 0; ww < PW_W; ++ww) {
-                if (ww == w) mine = pin;
-                const double tw = pin ? sh.tot[1][ww] : sh.tot[0][ww];
-                if (ww < w) Ew += tw;
-                T += tw;
-                const unsigned pm = sh.par[ww];
-                pin = (pm & 1u) ? (pin ^ (int)(pm >> 1)) : (int)(pm >> 1);
-            }
-            if (mine) E += (double)((int)__popcll(up1 & below) - (int)__popcll(dn1 & below));
-            E += Ew;
-            const double bf = seen ? (double)(base ^ (dep & mine) ^ g2) : 0.0;
-            const double lo = plo - E, up = phi - E;
-#pragma unroll
-            for (int i = 0; i < PW_R; ++i) {
-                q[i] += ((after >> i) & 1u) ? bf : 0.0;
-                if (!(q[i] > lo && q[i] < up)) flag |= 1u << i;
-            }
-            const uint64_t bal = __ballot(flag != 0);
-            if (bal) {
-                if (lane == __builtin_ctzll(bal)) {
-                    const int j = __builtin_ctz(flag);
-                    double before = E, vj = 0.0;
+                    const int fh = __builtin_ctz(halfm);
+                    after = ~0u << fh;
+                    double q0L = 0.0, add = 0.0;   // the prefix at the last tie; later rounding bits
 #pragma unroll
                     for (int i = 0; i < PW_R; ++i) {
-                        if (i < j) before = E + q[i];
-                        if (i == j) vj = v[i];
+                        const double q0 = q[i];
+                        if (i == fh) {
+                            g2 = pw_odd(q0);
+                            q0L = q0;
+                        } else if (i > fh && ((halfm >> i) & 1u)) {
+                            add += (double)pw_odd(q0 - q0L);
+                            q0L = q0;
+                        }
+                        q[i] = q0 + add;
                     }
-                    sh.brk_s[w] = (M + before) * u + vj;
-                    sh.brk_f[w] = f0 + j;
+                    gam = pw_odd(acc - q0L);
+                    acc = q[PW_R - 1];
                 }
-            } else if (lane == 0) {
-                sh.brk_f[w] = INT64_MAX;
+                // incoming parity of this lane: base ^ (dep & the wave's incoming parity)
+                const uint64_t Rm = __ballot(seen);
+                const uint64_t Xb = __ballot(gam);
+                const uint64_t Rb = Rm & below;
+                int base, dep;
+                if (Rb) {
+                    const int r = 63 - __clzll((long long)Rb);
+                    base = __popcll(Xb & below & ~((uint64_t(1) << r) - 1)) & 1;
+                    dep = 0;
+                } else {
+                    base = __popcll(Xb & below) & 1;
+                    dep = 1;
+                }
+                const int b0 = base ^ g2;   // the first halfway case's bit for an incoming parity 0
+                double incl;
+                double E = pw_wave_scan(acc + (seen ? (double)b0 : 0.0), incl);
+                // for an incoming parity 1 the lanes with seen && dep add 1 - 2*b0 instead of b0
+                // (counts as signed ints: __popcll is unsigned)
+                const uint64_t up1 = __ballot(seen && dep && !b0), dn1 = __ballot(seen && dep && b0);
+                if (lane == 63) {
+                    sh.tot[0][w] = incl;
+                    sh.tot[1][w] = incl + (double)((int)__popcll(up1) - (int)__popcll(dn1));
+                }
+                if (lane == 0) {
+                    int xw;
+                    if (Rm) {
+                        const int r = 63 - __clzll((long long)Rm);
+                        xw = __popcll(Xb & ~((uint64_t(1) << r) - 1)) & 1;
+                    } else {
+                        xw = __popcll(Xb) & 1;
+                    }
+                    sh.par[w] = (Rm ? 0u : 1u) | ((unsigned)xw << 1);
+                }
+                __syncthreads();
+                int pin = pw_odd(M), mine = 0;
+                double Ew = 0.0;
+#pragma unroll
+                for (int ww = 0; ww < PW_W; ++ww) {
+                    if (ww == w) mine = pin;
+                    const double tw = pin ? sh.tot[1][ww] : sh.tot[0][ww];
+                    if (ww < w) Ew += tw;
+                    T += tw;
+                    const unsigned pm = sh.par[ww];
+                    pin = (pm & 1u) ? (pin ^ (int)(pm >> 1)) : (int)(pm >> 1);
+                }
+                if (mine) E += (double)((int)__popcll(up1 & below) - (int)__popcll(dn1 & below));
+                E += Ew;
+                const double bf = seen ? (double)(base ^ (dep & mine) ^ g2) : 0.0;
+                const double lo = plo - E, up = phi - E;
+#pragma unroll
+                for (int i = 0; i < PW_R; ++i) {
+                    q[i] += ((after >> i) & 1u) ? bf : 0.0;
+                    if (!(q[i] > lo && q[i] < up)) flag |= 1u << i;
+                }
+                const uint64_t bal = __ballot(flag != 0);
+                if (bal) {
+                    if (lane == __builtin_ctzll(bal)) {
+                        const int j = __builtin_ctz(flag);
+                        double before = E, vj = 0.0;
+#pragma unroll
+                        for (int i = 0; i < PW_R; ++i) {
+                            if (i < j) before = E + q[i];
+                            if (i == j) vj = v[i];
+                        }
+                        sh.brk_s[w] = (M + before) * u + vj;
+                        sh.brk_f[w] = f0 + j;
+                    }
+                } else if (lane == 0) {
+                    sh.brk_f[w] = INT64_MAX;
+                }
+                __syncthreads();
             }
-            __syncthreads();
             int64_t bfi = INT64_MAX;
             double bs = 0.0;
 #pragma unroll
@@ -1379,7 +1401,7 @@ __device__ __forceinline__ double walk_plane_sum(const Geom& g, V value, PwShare
         }
         // chunk a+3 into the slot of chunk a-1, read from the round at a+2 on
         if (fetch) {
-            store_chunk(a + 3);
+            if (producer) store_chunk(a + 3);
             hi = a + 3;
         }
     }
@@ -1414,9 +1436,9 @@ __device__ __forceinline__ void plane_mean_body(const Geom& g, const TI* __restr
     if (threadIdx.x == 0) out[k * g.nz + z] = s / (double)(float)(g.nPx * g.nPy);
 }
 
-// PW_T threads per plane, the reference's order (walk_plane_sum).
+// PW_B threads per plane, the reference's order (walk_plane_sum).
 template <typename TI>
-__global__ void __launch_bounds__(PW_T)
+__global__ void __launch_bounds__(PW_B, 4)
 plane_mean_walk_kernel(Geom g, const TI* __restrict__ U, const double* __restrict__ bg64, int want_ro,
                        int want_tt, double* __restrict__ out)
 {

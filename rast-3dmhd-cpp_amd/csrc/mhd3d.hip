@@ -914,7 +914,7 @@ static int run_prepass_t(mhd3d_ctx* ctx, const TI* U, int stage, hipStream_t str
             plane_mean_tree_kernel<TI><<<grd, PT_T, 0, stream>>>(ctx->g, U, ctx->bg64, want_ro, want_tt,
                                                                  ctx->ext_buf);
         else
-            plane_mean_walk_kernel<TI><<<grd, PW_T, 0, stream>>>(ctx->g, U, ctx->bg64, want_ro, want_tt,
+            plane_mean_walk_kernel<TI><<<grd, PW_B, 0, stream>>>(ctx->g, U, ctx->bg64, want_ro, want_tt,
                                                                  ctx->ext_buf);
         HIPCHK(ctx, hipGetLastError());
     }
