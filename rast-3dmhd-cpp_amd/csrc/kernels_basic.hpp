@@ -761,8 +761,9 @@ __device__ __forceinline__ void wall_point(const StageArgs& a, int x, int y, boo
     }
 }
 
-// Wall planes of one RK stage as a separate launch (used with the point
-// kernel; the streaming kernel handles the walls of its own columns).
+// Wall planes of one RK stage as a launch of their own, after the interior's
+// (where the stage launch does not take them itself, see walls_in_stage); in
+// stage 3 it closes the step where e says so.
 // Latency-bound (two planes of one-sided stencils from global memory): built
 // for three waves per SIMD (FP64) or two (the mixed form's deviation
 // stencils), so the register allocator keeps the occupancy; the off-default

@@ -246,9 +246,8 @@ struct StageLds {
 };
 
 // One work item of a stage: the 32 x 8 tile (tile_x, tile_y) over the
-// interior planes zb .. ze-1 (the wall planes are a separate launch: their
-// one-sided stencils from global memory would raise this kernel's register
-// budget).  lds: StageLds::bytes of shared memory.  Stage 3 accumulates the
+// interior planes zb .. ze-1 (the wall planes follow in item_walls or in a
+// launch of their own).  lds: StageLds::bytes of shared memory.  Stage 3 accumulates the
 // CFL terms of every point it updates into cfl.
 // S32 (with T = double): the mixed form with the off-default branches --
 // fluxes evaluated in FP64 (with the branches) from the FP32 copies of the

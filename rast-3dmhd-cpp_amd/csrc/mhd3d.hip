@@ -6,8 +6,9 @@
 // read by stage 1 and rewritten by stage 3), the FP64 Z and two FP32 copies
 // of the stage values (written by stages 1 and 2, read by stages 2 and 3).
 // A step is: CFL (unless fixed DT or already evaluated inside the previous
-// stage 3) -> 3 x (interior stage kernel, wall stage kernel) -> clock update,
-// with DT kept on the device so the host never waits inside a step.
+// stage 3) -> 3 x (stage kernel, and the wall kernel where the stage kernel
+// does not take the walls), the last of them closing the step (clock, next
+// DT), with DT kept on the device so the host never waits inside a step.
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -676,7 +677,7 @@ extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
     // the other U buffers need the z ghost planes too (stage kernels never
     // write them)
-    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, upload_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, fields, ctx->U[ctx->cur],
                               ctx->mixed ? nullptr : ctx->U[1 - ctx->cur]));
     if (ctx->mixed) {
@@ -749,7 +750,7 @@ extern "C" int mhd3d_get_state(mhd3d_ctx* ctx, double* const* fields)
     if (!ctx || !fields) return MHD3D_EINVAL;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
-    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, download_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, ctx->U[ctx->cur], true, fields));
     return MHD3D_OK;
 }
@@ -1278,7 +1279,7 @@ extern "C" int mhd3d_fluxes(mhd3d_ctx* ctx, double* const* flux)
     else flux_only_kernel<false, false><<<grd, blk, 0, ctx->stream>>>(a, ctx->F);
     HIPCHK(ctx, hipGetLastError());
     // (the packing writes zeros for the ghosts, which nothing evaluates)
-    HIPCHK(ctx, staging_device(ctx->stage, &ctx->bytes));
+    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, download_fields(g, ctx->nf, ctx->stage, ctx->stream, ctx->F, false, flux));
     if (ctx->xa.flags & EXT_RLAX) {
         // the reference's fluxes() ends in exit_err at an exit point: the

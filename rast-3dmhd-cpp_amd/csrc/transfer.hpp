@@ -126,21 +126,27 @@ inline hipError_t staging_create(Staging& s, const Geom& g, int nf)
     return e;
 }
 
-// The device slabs where the transfers take them; *bytes grows by their size.
-inline hipError_t staging_device(Staging& s, int64_t* bytes)
+// The device slabs and the engine's stream where the transfers take them;
+// *bytes grows by their size.  Without room for them on the device the
+// transfers go through the pinned memory in place.
+inline void staging_device(Staging& s, int64_t* bytes)
 {
-    if (s.engine || s.slab_bytes < kDmaBytes) return hipSuccess;
+    if (s.engine || s.slab_bytes < kDmaBytes) return;
     hipError_t e = hipSuccess;
-    for (int k = 0; k < 2; ++k) {
-        if (e == hipSuccess && !s.dslab[k]) {
+    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
+        if (!s.dslab[k]) {
             e = hipMalloc(&s.dslab[k], s.slab_bytes);
-            if (e == hipSuccess) *bytes += (int64_t)s.slab_bytes;
+            if (e != hipSuccess) s.dslab[k] = nullptr;
+            else *bytes += (int64_t)s.slab_bytes;
         }
         if (e == hipSuccess && !s.kev[k]) e = hipEventCreateWithFlags(&s.kev[k], hipEventDisableTiming);
         if (e == hipSuccess && !s.dev_ev[k]) e = hipEventCreateWithFlags(&s.dev_ev[k], hipEventDisableTiming);
     }
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&s.engine, hipStreamNonBlocking);
-    return e;
+    if (e != hipSuccess) {
+        s.engine = nullptr;
+        (void)hipGetLastError();   // no error: later checks must not see it
+    }
 }
 
 inline void staging_destroy(Staging& s)
