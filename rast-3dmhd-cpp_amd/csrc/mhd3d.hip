@@ -677,7 +677,6 @@ extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
     // the other U buffers need the z ghost planes too (stage kernels never
     // write them)
-    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, upload_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, fields, ctx->U[ctx->cur],
                               ctx->mixed ? nullptr : ctx->U[1 - ctx->cur]));
     if (ctx->mixed) {
@@ -750,7 +749,6 @@ extern "C" int mhd3d_get_state(mhd3d_ctx* ctx, double* const* fields)
     if (!ctx || !fields) return MHD3D_EINVAL;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
-    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, download_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, ctx->U[ctx->cur], true, fields));
     return MHD3D_OK;
 }
@@ -1279,7 +1277,6 @@ extern "C" int mhd3d_fluxes(mhd3d_ctx* ctx, double* const* flux)
     else flux_only_kernel<false, false><<<grd, blk, 0, ctx->stream>>>(a, ctx->F);
     HIPCHK(ctx, hipGetLastError());
     // (the packing writes zeros for the ghosts, which nothing evaluates)
-    staging_device(ctx->stage, &ctx->bytes);
     HIPCHK(ctx, download_fields(g, ctx->nf, ctx->stage, ctx->stream, ctx->F, false, flux));
     if (ctx->xa.flags & EXT_RLAX) {
         // the reference's fluxes() ends in exit_err at an exit point: the

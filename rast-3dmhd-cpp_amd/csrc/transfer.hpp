@@ -10,13 +10,22 @@
 // helpers, started once for the call, take in turn; a helper that starts late
 // finds less to do and is never waited for before it has begun.
 //
-// Before, each field went in four slabs and each slab's rows were repacked by
-// up to 16 threads started for it, about 225 us a slab whatever its size.  ms
-// for get_state into kept arrays / set_state, before -> now, FP64 (MI355X; the
-// link moves 57 GB/s): hydro 32^3 (1.6 MB) 2.3 / 2.3 -> 0.08 / 0.10; 96x96x64
-// (25 MB) 5.6 / 4.8 -> 0.64 / 0.75; MHD 64^3 (18 MB) 7.5 / 7.0 -> 0.48 / 0.58;
-// 256x256x128 (554 MB) 14.2 / 13.2 -> 10.5 / 10.7; 512x512x256 (4.4 GB) 78 /
-// 82 -> 79 / 79.
+// The kernels read and write the pinned memory in place, at 52-53 of the
+// link's 57 GB/s.  Slabs of 8 MB and more went by the copy engine through two
+// device slabs before: its rate differs from machine to machine and from copy
+// to copy (512x512x256 get_state 78 ms at best, 146 at worst, and 97 for
+// set_state, against 83 and 83 in place whatever the machine), its set-up
+// slowed first transfers, and the device slabs came on top of a server's
+// budget.
+//
+// ms for get_state into kept arrays / set_state, FP64 (MI355X), a slab of rows
+// repacked by up to 16 threads started for it -> the copy engine -> now: hydro
+// 32^3 (1.6 MB) 2.3 / 2.3 -> 0.08 / 0.10 -> 0.08 / 0.11; MHD 64^3 (18 MB) 8.0 /
+// 7.7 -> 0.49 / 0.56 -> 0.49 / 0.57; 128^3 (141 MB) 9.0 / 8.8 -> 5.6 / 3.1 -> 3.1
+// / 3.2; 256x256x128 (554 MB) 18.7 / 14 -> 18.8 / 14 -> 11.1 / 10.9; 512x512x256
+// (4.4 GB) 146 / 84 -> 146 / 97 -> 83 / 83.  The first set_state of a context:
+// 128^3 9.3 -> 9.3 -> 8.4, 256x256x128 17.5 -> 20.7 -> 15.6, 512x512x256 104 -> 105
+// -> 89.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -81,32 +90,27 @@ MHD_TU_LOCAL __global__ void __launch_bounds__(256) unpack_planes_kernel(Geom g,
     }
 }
 
-// Staging of one domain: kSlabs pinned slabs of slab_planes planes.
+// Slabs of at most 24 MB: a context pins no more than 96 MB (unless one plane
+// is larger), and the first transfer has less memory to touch.  ms of the first
+// set_state / a fetch into fresh arrays at 512x512x256: slabs of 64 MB 95 /
+// 83.3, 32 MB 90 / 84.6, 24 MB 88 / 83.4, 16 MB 88 / 90, 8 MB 87 / 92 (too few
+// huge pages in flight for the helpers).
 constexpr int kSlabs = 4;
-constexpr size_t kSlabBytes = 64u << 20;   // at most, unless one plane is larger
+constexpr size_t kSlabBytes = 24u << 20;
 constexpr size_t kPieceBytes = 256u << 10; // the smallest host copy
 constexpr size_t kHugePage = 2u << 20;
 constexpr size_t kCallBytes = 64u << 10;
 constexpr size_t kHelperBytes = 2u << 20;  // a helper thread for each so many bytes
 
-// Slabs of at least kDmaBytes cross the link by the copy engine on a stream of
-// its own, through two device slabs that the kernels fill or empty meanwhile:
-// 56 GB/s against 52 for kernels that read and write the pinned memory in
-// place, which on small states saves the engine's start instead.
-constexpr size_t kDmaBytes = 8u << 20;
-
+// The slabs of one domain.
 struct Staging {
-    double* host = nullptr;   // pinned
-    double* dev = nullptr;    // its device address
-    double* dslab[2] = {};    // device slabs of large states, from the first transfer on
-    hipStream_t engine = nullptr;
-    hipEvent_t kev[2] = {}, dev_ev[2] = {};   // last kernel and last engine copy on each device slab
-    int slab_planes = 0;
-    size_t slab_bytes = 0;
-    hipEvent_t ev[kSlabs] = {};
+    double* host = nullptr;     // pinned, kSlabs slabs
+    double* dev = nullptr;      // its device address
+    hipEvent_t ev[kSlabs] = {}; // last kernel on each slab
 };
 
-// Planes per slab: a quarter of the state, within the slab limit.
+// Planes of a slab in the transfers of nf fields of g: a quarter of the
+// state, within the slab limit.
 inline int staging_planes(const Geom& g, int nf)
 {
     const size_t plane = (size_t)(g.nPx + 2) * (g.nPy + 2) * sizeof(double);
@@ -118,49 +122,18 @@ inline int staging_planes(const Geom& g, int nf)
 
 inline hipError_t staging_create(Staging& s, const Geom& g, int nf)
 {
-    s.slab_planes = staging_planes(g, nf);
-    s.slab_bytes = (size_t)s.slab_planes * (g.nPx + 2) * (g.nPy + 2) * sizeof(double);
-    hipError_t e = hipHostMalloc(&s.host, kSlabs * s.slab_bytes);
+    const size_t slab = (size_t)staging_planes(g, nf) * (g.nPx + 2) * (g.nPy + 2) * sizeof(double);
+    hipError_t e = hipHostMalloc(&s.host, kSlabs * slab);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&s.dev, s.host, 0);
     for (int k = 0; k < kSlabs && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
     return e;
 }
 
-// The device slabs and the engine's stream where the transfers take them;
-// *bytes grows by their size.  Without room for them on the device the
-// transfers go through the pinned memory in place.
-inline void staging_device(Staging& s, int64_t* bytes)
-{
-    if (s.engine || s.slab_bytes < kDmaBytes) return;
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        if (!s.dslab[k]) {
-            e = hipMalloc(&s.dslab[k], s.slab_bytes);
-            if (e != hipSuccess) s.dslab[k] = nullptr;
-            else *bytes += (int64_t)s.slab_bytes;
-        }
-        if (e == hipSuccess && !s.kev[k]) e = hipEventCreateWithFlags(&s.kev[k], hipEventDisableTiming);
-        if (e == hipSuccess && !s.dev_ev[k]) e = hipEventCreateWithFlags(&s.dev_ev[k], hipEventDisableTiming);
-    }
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s.engine, hipStreamNonBlocking);
-    if (e != hipSuccess) {
-        s.engine = nullptr;
-        (void)hipGetLastError();   // no error: later checks must not see it
-    }
-}
-
 inline void staging_destroy(Staging& s)
 {
-    if (s.engine) {
-        (void)hipStreamSynchronize(s.engine);
-        (void)hipStreamDestroy(s.engine);
-    }
-    for (hipEvent_t ev : {s.ev[0], s.ev[1], s.ev[2], s.ev[3], s.kev[0], s.kev[1], s.dev_ev[0], s.dev_ev[1]})
+    for (hipEvent_t ev : s.ev)
         if (ev) (void)hipEventDestroy(ev);
     if (s.host) (void)hipHostFree(s.host);
-    (void)hipFree(s.dslab[0]);
-    (void)hipFree(s.dslab[1]);
-    s = Staging{};
 }
 
 // Copies of numbered jobs, cut into pieces that the caller and the helpers
@@ -180,8 +153,8 @@ public:
             w.bytes = bytes[j];
             // a large job in pieces of whole huge pages of the caller's array,
             // so that no two threads first touch (and zero) the same page
-            const bool large = bytes[j] >= 16 * kHugePage;
-            w.piece = large ? kHugePage * std::max<size_t>(1, bytes[j] / (32 * kHugePage)) : kPieceBytes;
+            const bool large = bytes[j] >= 8 * kHugePage;
+            w.piece = large ? kHugePage : kPieceBytes;
             w.head = large ? heads[j] : 0;
             w.pieces = (w.bytes - w.head + w.piece - 1) / w.piece;
         }
@@ -265,12 +238,12 @@ struct ChunkPlan {
     int planes(int c) const { return std::min(total, (c + 1) * per) - c * per; }
 };
 
-inline ChunkPlan chunk_plan(const Geom& g, int nf, const Staging& s)
+inline ChunkPlan chunk_plan(const Geom& g, int nf)
 {
     ChunkPlan p;
     p.plane = (int64_t)(g.nPx + 2) * (g.nPy + 2);
     p.total = nf * g.nz;
-    p.per = s.slab_planes;
+    p.per = staging_planes(g, nf);
     p.n = (p.total + p.per - 1) / p.per;
     return p;
 }
@@ -324,11 +297,12 @@ inline int transfer_grid(int64_t n) { return (int)std::min<int64_t>((n + 255) / 
 inline hipError_t upload_fields(const Geom& g, int nf, Staging& s, hipStream_t stream, const double* const* src,
                                 double* U, double* V)
 try {
+    hipError_t e = hipSuccess;
     for (hipEvent_t ev : s.ev) {   // no earlier chunk is still on its way through a slab
-        const hipError_t e = hipEventSynchronize(ev);
+        e = hipEventSynchronize(ev);
         if (e != hipSuccess) return e;
     }
-    const ChunkPlan p = chunk_plan(g, nf, s);
+    const ChunkPlan p = chunk_plan(g, nf);
     std::vector<size_t> bytes, heads;
     chunk_sizes(p, g, src, bytes, heads);
     auto slab = [&](double* base, int c) { return base + (size_t)(c % kSlabs) * p.per * p.plane; };
@@ -341,29 +315,15 @@ try {
                   });
     for (int c = 0; c < p.n; ++c) {
         if (c >= kSlabs) {
-            const hipError_t e = hipEventSynchronize(s.ev[c % kSlabs]);   // the slab's last chunk is on the device
+            e = hipEventSynchronize(s.ev[c % kSlabs]);   // the slab's last chunk is on the device
             if (e != hipSuccess) return e;
         }
         team.open(c);
         team.finish(c);
-        const int d = c & 1;
-        hipError_t e = hipSuccess;
-        auto unpack = [&](const double* from) {
-            unpack_planes_kernel<<<transfer_grid(g.plane * p.planes(c)), 256, 0, stream>>>(g, from, p.begin(c),
+        unpack_planes_kernel<<<transfer_grid(g.plane * p.planes(c)), 256, 0, stream>>>(g, slab(s.dev, c), p.begin(c),
                                                                                        p.planes(c), U, V);
-            return hipGetLastError();
-        };
-        if (s.engine) {
-            if (c >= 2) e = hipStreamWaitEvent(s.engine, s.kev[d], 0);   // the device slab has been unpacked
-            if (e == hipSuccess) e = hipMemcpyAsync(s.dslab[d], slab(s.host, c), bytes[c], hipMemcpyHostToDevice, s.engine);
-            if (e == hipSuccess) e = hipEventRecord(s.ev[c % kSlabs], s.engine);
-            if (e == hipSuccess) e = hipStreamWaitEvent(stream, s.ev[c % kSlabs], 0);
-            if (e == hipSuccess) e = unpack(s.dslab[d]);
-            if (e == hipSuccess) e = hipEventRecord(s.kev[d], stream);
-        } else {
-            e = unpack(slab(s.dev, c));
-            if (e == hipSuccess) e = hipEventRecord(s.ev[c % kSlabs], stream);
-        }
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(s.ev[c % kSlabs], stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -375,27 +335,19 @@ try {
 inline hipError_t download_fields(const Geom& g, int nf, Staging& s, hipStream_t stream, const double* U,
                                   bool periodic, double* const* dst)
 try {
-    const ChunkPlan p = chunk_plan(g, nf, s);
+    const ChunkPlan p = chunk_plan(g, nf);
+    hipError_t e = hipSuccess;
     std::vector<size_t> bytes, heads;
     chunk_sizes(p, g, dst, bytes, heads);
     auto slab = [&](double* base, int c) { return base + (size_t)(c % kSlabs) * p.per * p.plane; };
     auto issue = [&](int c) -> hipError_t {
-        const int d = c & 1;
-        hipError_t e = hipSuccess;
-        if (s.engine && c >= 2) e = hipStreamWaitEvent(stream, s.dev_ev[d], 0);   // the device slab has gone out
-        if (e != hipSuccess) return e;
-        pack_planes_kernel<<<transfer_grid(p.plane * p.planes(c)), 256, 0, stream>>>(
-            g, U, p.begin(c), p.planes(c), periodic ? 1 : 0, s.engine ? s.dslab[d] : slab(s.dev, c));
-        e = hipGetLastError();
-        if (!s.engine) return e != hipSuccess ? e : hipEventRecord(s.ev[c % kSlabs], stream);
-        if (e == hipSuccess) e = hipEventRecord(s.kev[d], stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(s.engine, s.kev[d], 0);
-        if (e == hipSuccess) e = hipMemcpyAsync(slab(s.host, c), s.dslab[d], bytes[c], hipMemcpyDeviceToHost, s.engine);
-        if (e == hipSuccess) e = hipEventRecord(s.dev_ev[d], s.engine);
-        return e != hipSuccess ? e : hipEventRecord(s.ev[c % kSlabs], s.engine);
+        pack_planes_kernel<<<transfer_grid(p.plane * p.planes(c)), 256, 0, stream>>>(g, U, p.begin(c), p.planes(c),
+                                                                                     periodic ? 1 : 0, slab(s.dev, c));
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : hipEventRecord(s.ev[c % kSlabs], stream);
     };
     for (int c = 0; c < std::min(p.n, kSlabs); ++c) {
-        const hipError_t e = issue(c);
+        e = issue(c);
         if (e != hipSuccess) return e;
     }
     CopyTeam team(bytes, heads, transfer_helpers((size_t)p.total * p.plane * sizeof(double)),
@@ -413,7 +365,7 @@ try {
                   });
     int opened = 0;
     for (int c = 0; c < p.n; ++c) {
-        hipError_t e = hipSuccess;
+        e = hipSuccess;
         if (opened == c) {
             e = hipEventSynchronize(s.ev[c % kSlabs]);
             if (e != hipSuccess) return e;

@@ -1,10 +1,11 @@
 """Host transfers of the state and of the fluxes: what goes in comes back, bit
 for bit, with the x and y ghosts periodic, for states of one chunk, of several
-chunks, with planes split over fields and (through the copy engine) large
+chunks, with planes split over fields and more chunks than slabs for large
 ones; z ghost planes included."""
 import numpy as np
 import pytest
 
+from mhd3d import _lib as L
 from mhd3d.desc import Descriptor
 from mhd3d.domain import Domain
 from mhd3d.initial import periodic_fill, stratified_config
@@ -56,3 +57,20 @@ def test_flux_ghosts_are_zero(n):
         for a in dom.fluxes().values():
             inner = a[1:-1, 1:-1, 1:-1]
             assert np.isfinite(inner).all() and np.count_nonzero(a) == np.count_nonzero(inner)
+
+
+@pytest.mark.parametrize("n", [(60, 50, 40), (200, 190, 70)])
+def test_transfers_take_no_device_memory(n):
+    """A served run's device bytes are its registers, whatever is fetched: the
+    transfers allocate nothing on the device, also where the state fills the
+    ring of slabs several times (its chunks then straddle fields)."""
+    print(f"no device memory {n}", flush=True)
+    desc = Descriptor(stratified_config(*n, lMag=True))
+    with Domain(desc) as dom:
+        before = L.lib().mhd3d_device_bytes(dom.h)
+        for seed in (5, 6):
+            st = _random(desc, seed)
+            dom.set_state(st)
+            got = dom.state()
+            assert all(np.array_equal(st[k].view(np.int64), got[k].view(np.int64)) for k in st)
+        assert L.lib().mhd3d_device_bytes(dom.h) == before
