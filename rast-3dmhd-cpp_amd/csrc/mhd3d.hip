@@ -52,7 +52,8 @@ struct mhd3d_ctx {
     CflPart* cfl_parts = nullptr;
     int cfl_parts_cap = 0;
     bool dt_ready = false;          // ds->dt holds TSTEP of the current state
-    Staging stage;                  // pinned slabs of the host transfers
+    Staging own_stage;              // of the host transfers
+    Staging* stage = &own_stage;    // its own, or its ensemble's or server's
     hipStream_t stream = nullptr;
     int cur = 0;
     int device = 0;
@@ -465,8 +466,7 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
     if (hipMalloc(&ctx->ds, sizeof(DevScalars)) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(scalars) failed");
     if (hipMemset(ctx->Z, 0, reg) != hipSuccess || hipMemset(ctx->ds, 0, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_EHIP, "hipMemset failed");
-    if (staging_create(ctx->stage, g, ctx->nf) != hipSuccess ||
-        hipHostMalloc(&ctx->hs, sizeof(DevScalars)) != hipSuccess)
+    if (hipHostMalloc(&ctx->hs, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_ENOMEM, "hipHostMalloc failed");
     ctx->bytes += (int64_t)((nU64 + 1) * reg + (ctx->mixed ? 2 * reg32 : 0) + nmet * sizeof(double) +
                             sizeof(DevScalars));
@@ -524,7 +524,7 @@ extern "C" int mhd3d_destroy(mhd3d_ctx* ctx)
     (void)hipFree(ctx->ft);
     (void)hipFree(ctx->relax_buf);
     (void)hipFree(ctx->rs);
-    staging_destroy(ctx->stage);
+    staging_destroy(ctx->own_stage);
     if (ctx->hs) (void)hipHostFree(ctx->hs);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -669,15 +669,29 @@ static int set_background_profiles(mhd3d_ctx* ctx, const std::vector<double>* me
     return MHD3D_OK;
 }
 
+// A transfer through the context's staging, which the members of an ensemble
+// share: one at a time, and nothing of it is under way when the next begins.
+struct Transfer {
+    mhd3d_ctx* ctx;
+    std::lock_guard<std::mutex> lock;
+    bool over = false;   // the stream has drained; otherwise (an error) the destructor waits for it
+    explicit Transfer(mhd3d_ctx* c) : ctx(c), lock(c->stage->mu) {}
+    ~Transfer()
+    {
+        if (!over) (void)hipStreamSynchronize(ctx->stream);
+    }
+};
+
 extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
 {
     if (!ctx || !fields) return MHD3D_EINVAL;
     ctx->dt_ready = false;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
+    Transfer hold(ctx);
     // the other U buffers need the z ghost planes too (stage kernels never
     // write them)
-    HIPCHK(ctx, upload_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, fields, ctx->U[ctx->cur],
+    HIPCHK(ctx, upload_fields(ctx->g, ctx->nf, *ctx->stage, ctx->stream, fields, ctx->U[ctx->cur],
                               ctx->mixed ? nullptr : ctx->U[1 - ctx->cur]));
     if (ctx->mixed) {
         int rc = set_background(ctx, fields);
@@ -692,6 +706,7 @@ extern "C" int mhd3d_set_state(mhd3d_ctx* ctx, const double* const* fields)
     ctx->relax_exit_seen = false;
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    hold.over = true;
     return MHD3D_OK;
 }
 
@@ -749,7 +764,9 @@ extern "C" int mhd3d_get_state(mhd3d_ctx* ctx, double* const* fields)
     if (!ctx || !fields) return MHD3D_EINVAL;
     for (int f = 0; f < ctx->nf; ++f)
         if (!fields[f]) return fail(ctx, MHD3D_EINVAL, "null field pointer");
-    HIPCHK(ctx, download_fields(ctx->g, ctx->nf, ctx->stage, ctx->stream, ctx->U[ctx->cur], true, fields));
+    Transfer hold(ctx);
+    HIPCHK(ctx, download_fields(ctx->g, ctx->nf, *ctx->stage, ctx->stream, ctx->U[ctx->cur], true, fields));
+    hold.over = true;   // the last chunk has arrived
     return MHD3D_OK;
 }
 
@@ -1277,7 +1294,11 @@ extern "C" int mhd3d_fluxes(mhd3d_ctx* ctx, double* const* flux)
     else flux_only_kernel<false, false><<<grd, blk, 0, ctx->stream>>>(a, ctx->F);
     HIPCHK(ctx, hipGetLastError());
     // (the packing writes zeros for the ghosts, which nothing evaluates)
-    HIPCHK(ctx, download_fields(g, ctx->nf, ctx->stage, ctx->stream, ctx->F, false, flux));
+    {
+        Transfer hold(ctx);
+        HIPCHK(ctx, download_fields(g, ctx->nf, *ctx->stage, ctx->stream, ctx->F, false, flux));
+        hold.over = true;
+    }
     if (ctx->xa.flags & EXT_RLAX) {
         // the reference's fluxes() ends in exit_err at an exit point: the
         // fluxes are complete, then the domain stops
@@ -1567,6 +1588,7 @@ struct mhd3d_ensemble {
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int64_t cells = 0;
     std::vector<DevScalars> last;      // members' scalars after the last step call
+    Staging stage;                     // of the members' host transfers
     std::string err;
 };
 
@@ -1850,6 +1872,7 @@ extern "C" int mhd3d_ensemble_create(const mhd3d_desc* const* descs, int n, mhd3
         int rc = mhd3d_create(descs[m], &c);
         if (rc) return bail(rc, "member " + std::to_string(m) + ": " + g_create_error);
         c->kernel_mode = 0;
+        c->stage = &e->stage;
         e->mem.push_back(c);
         e->cells += (int64_t)descs[m]->nPx * descs[m]->nPy * descs[m]->nPz;
     }
@@ -1869,6 +1892,7 @@ extern "C" int mhd3d_ensemble_destroy(mhd3d_ensemble* e)
     ens_drop_graphs(e);
     if (e->owns)
         for (auto* c : e->mem) mhd3d_destroy(c);
+    staging_destroy(e->stage);
     (void)hipFree(e->mirror);
     (void)hipFree(e->d_items);
     (void)hipFree(e->d_items_x);
@@ -2299,6 +2323,7 @@ struct mhd3d_server {
     int64_t budget = 0, used = 0;
     int quantum = 10;
     mhd3d_ensemble* ens = nullptr;    // view over the admitted runs (owns = false)
+    Staging stage;                    // of the runs' fetches
     std::unordered_map<int64_t, ServerReq> reqs;
     std::deque<int64_t> queue;
     std::vector<int64_t> active;
@@ -2363,6 +2388,7 @@ extern "C" int mhd3d_server_destroy(mhd3d_server* s)
     if (s->ens) mhd3d_ensemble_destroy(s->ens);   // a view: leaves the runs
     for (auto& kv : s->reqs)
         if (kv.second.ctx) mhd3d_destroy(kv.second.ctx);
+    staging_destroy(s->stage);
     delete s;
     return MHD3D_OK;
 }
@@ -2447,6 +2473,7 @@ static int srv_admit(mhd3d_server* s)
         mhd3d_ctx* c = nullptr;
         int rc = mhd3d_create(&r.d, &c);
         if (rc) { s->err = g_create_error; return rc; }
+        c->stage = &s->stage;
         rc = mhd3d_init_stratified(c, r.Tz.data(), r.Rz.data(), r.seed, r.amp, r.b0, r.b_amp);
         if (!rc) rc = mhd3d_set_dt_guard(c, MHD3D_REFERENCE_DT_MIN);
         if (!rc) {

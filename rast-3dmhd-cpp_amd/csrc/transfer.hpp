@@ -102,10 +102,14 @@ constexpr size_t kHugePage = 2u << 20;
 constexpr size_t kCallBytes = 64u << 10;
 constexpr size_t kHelperBytes = 2u << 20;  // a helper thread for each so many bytes
 
-// The slabs of one domain.
+// The slabs and what goes with them: a domain's own, or one that the members
+// of an ensemble or the runs of a server take in turn.  Nothing is allocated
+// before the first transfer.
 struct Staging {
+    std::mutex mu;              // held for the length of a transfer
     double* host = nullptr;     // pinned, kSlabs slabs
     double* dev = nullptr;      // its device address
+    size_t slab_bytes = 0;      // allocated for each
     hipEvent_t ev[kSlabs] = {}; // last kernel on each slab
 };
 
@@ -120,12 +124,20 @@ inline int staging_planes(const Geom& g, int nf)
     return (int)n;
 }
 
-inline hipError_t staging_create(Staging& s, const Geom& g, int nf)
+// Room for slabs of `want` bytes; no transfer is under way.
+inline hipError_t staging_reserve(Staging& s, size_t want)
 {
-    const size_t slab = (size_t)staging_planes(g, nf) * (g.nPx + 2) * (g.nPy + 2) * sizeof(double);
-    hipError_t e = hipHostMalloc(&s.host, kSlabs * slab);
-    if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&s.dev, s.host, 0);
-    for (int k = 0; k < kSlabs && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < kSlabs && e == hipSuccess; ++k)
+        if (!s.ev[k]) e = hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
+    if (e != hipSuccess || s.slab_bytes >= want) return e;
+    if (s.host) (void)hipHostFree(s.host);
+    s.host = s.dev = nullptr;
+    s.slab_bytes = 0;
+    e = hipHostMalloc(&s.host, kSlabs * want);
+    if (e != hipSuccess) s.host = nullptr;
+    else e = hipHostGetDevicePointer((void**)&s.dev, s.host, 0);
+    if (e == hipSuccess) s.slab_bytes = want;
     return e;
 }
 
@@ -234,6 +246,7 @@ struct ChunkPlan {
     int64_t plane;             // doubles of one host plane
     int total, per;
     int n;
+    size_t slab() const { return (size_t)per * plane * sizeof(double); }
     int begin(int c) const { return c * per; }
     int planes(int c) const { return std::min(total, (c + 1) * per) - c * per; }
 };
@@ -293,16 +306,13 @@ inline void chunk_sizes(const ChunkPlan& p, const Geom& g, P const* fields, std:
 inline int transfer_grid(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 2048); }
 
 // The host's fields into register U (and V).  The stream orders the kernels;
-// the caller synchronizes it before the staging is used again.
+// the caller holds the staging until the stream has drained.
 inline hipError_t upload_fields(const Geom& g, int nf, Staging& s, hipStream_t stream, const double* const* src,
                                 double* U, double* V)
 try {
-    hipError_t e = hipSuccess;
-    for (hipEvent_t ev : s.ev) {   // no earlier chunk is still on its way through a slab
-        e = hipEventSynchronize(ev);
-        if (e != hipSuccess) return e;
-    }
     const ChunkPlan p = chunk_plan(g, nf);
+    hipError_t e = staging_reserve(s, p.slab());
+    if (e != hipSuccess) return e;
     std::vector<size_t> bytes, heads;
     chunk_sizes(p, g, src, bytes, heads);
     auto slab = [&](double* base, int c) { return base + (size_t)(c % kSlabs) * p.per * p.plane; };
@@ -336,7 +346,8 @@ inline hipError_t download_fields(const Geom& g, int nf, Staging& s, hipStream_t
                                   bool periodic, double* const* dst)
 try {
     const ChunkPlan p = chunk_plan(g, nf);
-    hipError_t e = hipSuccess;
+    hipError_t e = staging_reserve(s, p.slab());
+    if (e != hipSuccess) return e;
     std::vector<size_t> bytes, heads;
     chunk_sizes(p, g, dst, bytes, heads);
     auto slab = [&](double* base, int c) { return base + (size_t)(c % kSlabs) * p.per * p.plane; };
