@@ -644,9 +644,9 @@ __device__ __forceinline__ void item_walls(const StageArgs& a, int tile_x, int t
 // the two planes BCON reads, take their columns' wall points as well (the
 // lean ones, see wall_point) and a stage-3 launch closes the step: one launch
 // per stage.  See walls_in_stage for where that pays.  Built for the default
-// variants only (default_variant), which need no accumulation registers; a
-// build of the mixed (1 wave, undeferred) variant that spilled to them
-// flagged finite states as non-finite.
+// variants only (default_waves, default_sched), whose values fit the vector
+// registers; the build refuses one that needs accumulation registers or
+// scratch memory (check_walls in build.py has the reason).
 template <typename T, bool MAG, bool ROT, int STAGE, int WAVES, bool ONE_BARRIER, bool DEFER,
           bool EXT = false, int EXTM = EXT_INTERIOR, bool S32 = false, bool WALLS = false>
 __global__ void __launch_bounds__(256, WAVES) stage_stream_kernel(StageArgs a, int zchunk, int nch, int ntx, int nty,
