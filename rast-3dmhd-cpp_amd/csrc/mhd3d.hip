@@ -358,11 +358,19 @@ static int variant_resident(const mhd3d_ctx* ctx, int w, int sc)
 // their columns in the stage launch.  Where the launch is one round of the
 // resident blocks, a wall launch after it is idle time (FP64, us a step, walls
 // apart -> in the stage: hydro 32^3 47 -> 37, MHD 64^3 85 -> 70, 96x96x64 141
-// -> 132, 256x256x128 1235 -> 1216); with more rounds the first and last
-// chunks' longer blocks cost more than the launch (192x192x96 602 -> 612,
-// 512x512x256 10057 -> 10211).  The mixed form's wall code slows its
-// stages (128x128x64 179 -> 181, 512x512x256 8.67 -> 8.84 ms), so there only
-// for chunks of a few planes (64^3 80 -> 74).
+// -> 132; of 84 hydro and MHD grids from 24x24x40 to 320x200x40 and 256x256x128
+// most are 3-15% faster so, two slower by 0.4 and 0.8%); with more rounds the first
+// and last chunks' longer blocks cost more than the launch (192x192x96 602 ->
+// 612, 512x512x256 10057 -> 10211).  The mixed form's wall code slows its
+// stages, and a chunk's blocks run side by side on one XCD: with 16 chunks and
+// more, those with walls are at most half of its blocks (MHD, 22 grids of 1 to
+// 5 planes a chunk: 2-12% faster; 64^3 77.3 -> 73.3, 64x64x128 108.2 -> 102.4),
+// with fewer they are most of them (28 grids: 0-6% slower but for one; 128x128x20
+// 92.2 -> 97.7, 96x96x32 90.4 -> 93.0, 101x75x37 even, 128x128x64 177.5 ->
+// 180.5).  Its hydro stages gain with fewer chunks too while those are short
+// (up to 3 planes and a remainder: 0-16% faster; 128x128x24 66.7 -> 61.8; 4
+// planes: 160x160x24 92.2 -> 97.2; 7: 128x128x64 118.4 -> 120.1).  512x512x256:
+// 8.67 -> 8.84 ms.
 static bool walls_in_stage(const mhd3d_ctx* ctx, int resident)
 {
     if (!ctx->ends || walls_full(ctx->d)) return false;
@@ -372,7 +380,8 @@ static bool walls_in_stage(const mhd3d_ctx* ctx, int resident)
         return false;   // the wall code is built into the default variants
     const StreamPlan p = stream_plan(ctx->g, ctx->target_blocks);
     if (p.nblocks > resident) return false;
-    return !ctx->mixed || p.zchunk < 4;
+    if (!ctx->mixed) return true;
+    return (p.nchunks >= 16 && p.zchunk < 6) || (ph == 0 && p.zchunk < 4);
 }
 
 extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)

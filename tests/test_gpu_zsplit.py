@@ -42,3 +42,24 @@ def test_mixed_split_changes_nothing(monkeypatch):
             out.append(dom.state())
     for k in out[0]:
         assert np.array_equal(out[0][k].view(np.int64), out[1][k].view(np.int64)), k
+
+
+@pytest.mark.parametrize("mag", [False, True])
+@pytest.mark.parametrize("n", [(64, 16, 150), (64, 64, 160), (64, 64, 200), (96, 96, 32), (128, 128, 20), (160, 160, 24)])
+def test_mixed_walls_in_the_stage_or_apart(monkeypatch, n, mag):
+    """The mixed form on both sides of the line that puts the walls into the
+    stage launch (chunks and planes a chunk), against a variant that launches
+    its walls apart: the same bits."""
+    print(f"mixed walls {n} mag={mag}", flush=True)
+    desc = Descriptor(stratified_config(*n, lMag=mag, lRot=True, precision=1))
+    st = stratified_state(desc, seed=4)
+    out = []
+    for variant in (None, "1,0"):
+        if variant:
+            monkeypatch.setenv("MHD3D_TUNE_MIXED_MHD" if mag else "MHD3D_TUNE_MIXED_HYDRO", variant)
+        with Domain(desc) as dom:
+            dom.set_state(st)
+            out.append((dom.step(3), dom.state()))
+    assert out[0][0] == out[1][0]
+    for k in out[0][1]:
+        assert np.array_equal(out[0][1][k].view(np.int64), out[1][1][k].view(np.int64)), k
