@@ -297,7 +297,7 @@ static int setup_ext(mhd3d_ctx* ctx, const mhd3d_desc* d)
         // FT is a static array of the reference, zero at program start
         const size_t bytes = (size_t)g.fs * sizeof(double);
         HIPCHK(ctx, hipMalloc(&ctx->ft, bytes));
-        HIPCHK(ctx, hipMemset(ctx->ft, 0, bytes));
+        HIPCHK(ctx, hipMemsetAsync(ctx->ft, 0, bytes, ctx->stream));
         ctx->bytes += (int64_t)bytes;
         X.ft = ctx->ft;
     }
@@ -453,27 +453,30 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
     const size_t reg = (size_t)g.fs * ctx->nf * sizeof(double);
     const size_t reg32 = (size_t)g.fs * ctx->nf * sizeof(float);
     const int nU64 = ctx->mixed ? 1 : 2;
+    // cleared on the context's own stream: it does not wait for the default
+    // one, where hipMemset returns before the memory is cleared
+    auto clear = [&](void* p, size_t bytes) { return hipMemsetAsync(p, 0, bytes, ctx->stream); };
     for (int k = 0; k < nU64; ++k) {
         if (hipMalloc(&ctx->U[k], reg) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(U) failed");
-        if (hipMemset(ctx->U[k], 0, reg) != hipSuccess) return cleanup(MHD3D_EHIP, "hipMemset failed");
+        if (clear(ctx->U[k], reg) != hipSuccess) return cleanup(MHD3D_EHIP, "hipMemset failed");
     }
     if (ctx->mixed) {
         for (int k = 0; k < 2; ++k) {
             if (hipMalloc(&ctx->U32[k], reg32) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(U32) failed");
-            if (hipMemset(ctx->U32[k], 0, reg32) != hipSuccess) return cleanup(MHD3D_EHIP, "hipMemset failed");
+            if (clear(ctx->U32[k], reg32) != hipSuccess) return cleanup(MHD3D_EHIP, "hipMemset failed");
         }
         if (hipMalloc(&ctx->bgf, sizeof(float) * NBGF * nz) != hipSuccess ||
             hipMalloc(&ctx->bg64, sizeof(double) * NBG64 * nz) != hipSuccess)
             return cleanup(MHD3D_ENOMEM, "hipMalloc(background) failed");
-        if (hipMemset(ctx->bgf, 0, sizeof(float) * NBGF * nz) != hipSuccess ||
-            hipMemset(ctx->bg64, 0, sizeof(double) * NBG64 * nz) != hipSuccess)
+        if (clear(ctx->bgf, sizeof(float) * NBGF * nz) != hipSuccess ||
+            clear(ctx->bg64, sizeof(double) * NBG64 * nz) != hipSuccess)
             return cleanup(MHD3D_EHIP, "hipMemset failed");
         ctx->h_dzz.assign(desc->dzzdz, desc->dzzdz + nz);
         ctx->h_d2zz.assign(desc->d2zzdz2, desc->d2zzdz2 + nz);
     }
     if (hipMalloc(&ctx->Z, reg) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(Z) failed");
     if (hipMalloc(&ctx->ds, sizeof(DevScalars)) != hipSuccess) return cleanup(MHD3D_ENOMEM, "hipMalloc(scalars) failed");
-    if (hipMemset(ctx->Z, 0, reg) != hipSuccess || hipMemset(ctx->ds, 0, sizeof(DevScalars)) != hipSuccess)
+    if (clear(ctx->Z, reg) != hipSuccess || clear(ctx->ds, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_EHIP, "hipMemset failed");
     if (hipHostMalloc(&ctx->hs, sizeof(DevScalars)) != hipSuccess)
         return cleanup(MHD3D_ENOMEM, "hipHostMalloc failed");
@@ -509,6 +512,8 @@ extern "C" int mhd3d_create(const mhd3d_desc* desc, mhd3d_ctx** out)
         ctx->ends = !ctx->ext && ctx->kernel_mode == 0;
         ctx->fold = walls_in_stage(ctx, res);
     }
+    // an ensemble or a server takes the context to a stream of its own
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return cleanup(MHD3D_EHIP, "clearing the registers failed");
     *out = ctx;
     return MHD3D_OK;
 }
