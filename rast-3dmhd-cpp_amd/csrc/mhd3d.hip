@@ -684,7 +684,8 @@ static int set_background_profiles(mhd3d_ctx* ctx, const std::vector<double>* me
 }
 
 // A transfer through the context's staging, which the members of an ensemble
-// share: one at a time, and nothing of it is under way when the next begins.
+// or the runs of a server share: one at a time, and nothing of it is under way
+// when the next begins.
 struct Transfer {
     mhd3d_ctx* ctx;
     std::lock_guard<std::mutex> lock;
